@@ -88,6 +88,19 @@ struct DSmoother {
   int gnx = 0, gny = 0, gnz = 0;
   V *lgs = nullptr, *ugs = nullptr, *dgs = nullptr, *tgs = nullptr, *xgs = nullptr;
   int64_t gsz = 0;
+  // Packed single-workgroup substitutions (mld_tripack.hpp): the packed
+  // factors, the U solve's input by position of the L solve (ILU), and two
+  // work vectors in position order; not built where the factors do not take
+  // that form
+  struct PackedTri {
+    unsigned char* pk = nullptr;  // null: not built
+    int* hdr = nullptr;
+    int* first = nullptr;
+    int ngroups = 0;
+    int *in = nullptr, *pos = nullptr;  // position -> row, row -> position
+  } lp, up;
+  int* ulin = nullptr;
+  V *tpa = nullptr, *tpb = nullptr;
   // dense LU
   double* lu = nullptr; int* piv = nullptr;
   double* dinv = nullptr;  // DENSE_LU: explicit inverse (row-major)

@@ -22,6 +22,7 @@
 #include "mld_dense.hpp"
 #include "mld_devcommon.hpp"
 #include "mld_kernels.hpp"
+#include "mld_tripack.hpp"
 
 namespace mld {
 
@@ -615,6 +616,7 @@ class DevPrecT : public DevPrec {
                          S.gnx, S.gny, S.gnz);
         }
       }
+      if (!S.lgs) packed_upload(H, S);
       HIPCHECK(hipStreamSynchronize(s_));
     }
     if (H.solver == DENSE_LU) {
@@ -625,6 +627,54 @@ class DevPrecT : public DevPrec {
       S.ndense = n;
       dense_factor_invert(n, S.lu, S.piv, S.dinv);
     }
+  }
+
+  // The packed single-workgroup form of the triangular factors (both of an
+  // ILU solver, the one that a Gauss-Seidel sweep solves with).
+  void packed_upload(const SmootherData& H, DSmoother<V>& S) {
+    const int n = H.l.nr;
+    if (n < TP_MIN_ROWS) return;
+    const bool ilu = (H.solver == ILU_N);
+    tp::Packed<V> pl, pu;
+    const double* d = H.dv.empty() ? nullptr : H.dv.data();
+    if ((ilu || H.solver == GS) && !tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl)) return;
+    if ((ilu || H.solver == BWGS) && !tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu)) return;
+    std::vector<int> pos(n), idx(n);
+    auto up = [&](const tp::Packed<V>& f, typename DSmoother<V>::PackedTri& t) {
+      for (int p = 0; p < n; ++p) pos[f.rows[p]] = p;
+      t.pk = ar_.upload(f.bytes.data(), f.bytes.size(), s_);
+      t.hdr = ar_.upload((const int*)f.hdr.data(), f.hdr.size() * 4, s_);
+      t.first = ar_.upload(f.first.data(), f.first.size(), s_);
+      t.in = ar_.upload(f.rows.data(), f.rows.size(), s_);
+      t.pos = ar_.upload(pos.data(), pos.size(), s_);
+      t.ngroups = f.ngroups;
+      HIPCHECK(hipStreamSynchronize(s_));
+    };
+    if (pl.ngroups) up(pl, S.lp);
+    if (ilu) {  // pos holds L's positions
+      for (int p = 0; p < n; ++p) idx[p] = pos[pu.rows[p]];
+      S.ulin = ar_.upload(idx.data(), idx.size(), s_);
+      HIPCHECK(hipStreamSynchronize(s_));
+    }
+    if (pu.ngroups) up(pu, S.up);
+    S.tpa = ar_.alloc<V>(n);
+    S.tpb = ar_.alloc<V>(n);
+    if (std::getenv("MLD_VERBOSE"))
+      std::fprintf(stderr, "[mld] %d-row factors packed for one workgroup: %d and %d groups, %zu and %zu level sets\n",
+                   n, pl.ngroups, pu.ngroups, H.lsched_ptr.size() - 1, H.usched_ptr.size() - 1);
+  }
+  static constexpr int TP_MIN_ROWS = 128;
+  static int tp_blocks(int n) { return (n + 255) / 256; }
+  template <int SC>
+  void tp_solve(const typename DSmoother<V>::PackedTri& f, V* bt) {
+    tp::tripack_kernel<V, SC><<<1, tp::TP_T, 0, s_>>>(f.ngroups, f.pk, (const tp::SliceHdr*)f.hdr, f.first, bt);
+    HIPCHECK(hipGetLastError());
+  }
+  void tp_out(int n, const int* pos, const V* s, V* t, V* y, int bt) {
+    if (bt == 0) tp::tripack_out<V, 0><<<tp_blocks(n), 256, 0, s_>>>(n, pos, s, t, y);
+    else if (bt == 1) tp::tripack_out<V, 1><<<tp_blocks(n), 256, 0, s_>>>(n, pos, s, t, y);
+    else tp::tripack_out<V, 2><<<tp_blocks(n), 256, 0, s_>>>(n, pos, s, t, y);
+    HIPCHECK(hipGetLastError());
   }
 
   // Blocked LU with partial pivoting (MFMA trailing updates) and the explicit
@@ -759,6 +809,14 @@ class DevPrecT : public DevPrec {
     const int* p1d = TR ? S.utptr_d : S.lptr_d;
     const int* p2d = TR ? S.ltptr_d : S.uptr_d;
     const int nl1 = (int)p1.size() - 1, nl2 = (int)p2.size() - 1;
+    if (!TR && S.lp.pk && S.up.pk && sync_free()) {
+      tp::tripack_in<V><<<tp_blocks(n), 256, 0, s_>>>(n, S.lp.in, x, S.tpa);
+      tp_solve<0>(S.lp, S.tpa);
+      tp::tripack_in<V><<<tp_blocks(n), 256, 0, s_>>>(n, S.ulin, S.tpa, S.tpb);
+      tp_solve<1>(S.up, S.tpb);
+      tp_out(n, S.up.pos, S.tpb, nullptr, y, beta ? 1 : 0);
+      return;
+    }
     V* t1 = D.tx;
     V* t2 = beta ? D.t2 : y;
     if (n <= SMALL_TRI) {
@@ -1076,6 +1134,13 @@ class DevPrecT : public DevPrec {
       else if (bt == 1) trsv_run_kernel<V, 2, 1, false, LN><<<1, 1024, 0, s_>>>(l0, l1, pd, rows, T.irp, T.ja, T.val, b, S.dv, t, y);
       else trsv_run_kernel<V, 2, 2, false, LN><<<1, 1024, 0, s_>>>(l0, l1, pd, rows, T.irp, T.ja, T.val, b, S.dv, t, y);
     };
+    const auto& pt = lower ? S.lp : S.up;
+    if (pt.pk && sync_free()) {
+      tp::tripack_in<V><<<tp_blocks(D.n), 256, 0, s_>>>(D.n, pt.in, b, S.tpa);
+      tp_solve<2>(pt, S.tpa);
+      tp_out(D.n, pt.pos, S.tpa, bt == 2 ? t : nullptr, y, bt);
+      return;
+    }
     if (D.n <= SMALL_TRI) {  // whole solve in one workgroup
       run(0, nl);
       return;
