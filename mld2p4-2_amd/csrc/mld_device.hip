@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
+#include <future>
 #include <cstdio>
 #include <thread>
 #include <cstdlib>
@@ -22,6 +23,7 @@
 #include "mld_dense.hpp"
 #include "mld_devcommon.hpp"
 #include "mld_kernels.hpp"
+#include "mld_tail.hpp"
 #include "mld_tripack.hpp"
 
 namespace mld {
@@ -115,17 +117,27 @@ class DevPrecT : public DevPrec {
     return 0;
   }
 
-  // Dense tail: from the first level l >= 1 with at most DENSE_TAIL_MAX rows,
-  // the untransposed cycle on levels l .. nlev-1 is a fixed linear operator
-  // B_l of x2l (no K-cycle there), formed once here by applying that cycle to
-  // the unit vectors and applied afterwards as one dense product
-  // y2l = B_l x2l: about ten launches of a few microseconds each become one.
-  // 'T' applications keep the level-by-level cycle.  Not taken when that
-  // level is a coarsest level already solved by one dense product
-  // (DENSE_LU), nor with MLD_DENSE_TAIL=0.  Same operator; the sums of the
-  // product are rounded in another order.
+  // Dense tail: from a level l >= 1 on, the untransposed cycle on levels
+  // l .. nlev-1 is a fixed linear operator B_l of x2l (no K-cycle there),
+  // formed once here and applied afterwards as one dense product y2l = B_l
+  // x2l: about ten launches of a few microseconds each become one.  'T'
+  // applications keep the level-by-level cycle.  Not taken when that level is
+  // a coarsest level already solved by one dense product (DENSE_LU), nor with
+  // MLD_DENSE_TAIL=0.  Same operator; the sums of the product are rounded in
+  // another order.
+  // The first level of at most DENSE_TAIL_MAX rows, or a larger one where its
+  // n^2 values are at most 16 per entry of the fine matrix, so that reading
+  // them stays a small part of the cycle's traffic, and take at most
+  // DENSE_TAIL_BYTES (Jacobi-type smoothers: about 30 us level by level; with
+  // 82 MB, 3195 rows in FP64 below a 101^3 grid, a V-cycle takes 186 us
+  // against 184, with 36 MB, below 93^3, a CG iteration 214 against 229) or
+  // DENSE_TAIL_BYTES_TRI where a level has triangular solves (2349 rows below
+  // a 96^3 grid with ILU(0): 3.3 ms per cycle in one workgroup, 1.2 ms packed,
+  // 10 us as one product).
   static constexpr int DENSE_TAIL_MAX = 1024;
+  static constexpr double DENSE_TAIL_BYTES = 48e6, DENSE_TAIL_BYTES_TRI = 134.3e6;
   int tail_lev_ = -1;
+  int tail_ld_ = 0;
   V* tail_b_ = nullptr;
   void build_tail() {
     tail_lev_ = -1;
@@ -133,29 +145,86 @@ class DevPrecT : public DevPrec {
     if (const char* e = std::getenv("MLD_DENSE_TAIL"))
       if (e[0] == '0') return;
     const int nlev = (int)L_.size();
+    const double few = 16.0 * (double)hprec_->precv[0].a.nnz();
+    auto fits = [&](int l) {
+      const double n2 = (double)L_[l].n * L_[l].n;
+      bool tri = false;
+      for (int k = l; k + 1 < nlev; ++k)
+        for (int sv : {L_[k].sm.solver, L_[k].has_sm2 ? L_[k].sm2.solver : (int)F_NONE})
+          tri = tri || sv == ILU_N || sv == GS || sv == BWGS;
+      return L_[l].n <= DENSE_TAIL_MAX ||
+             (n2 <= few && n2 * sizeof(V) <= (tri ? DENSE_TAIL_BYTES_TRI : DENSE_TAIL_BYTES));
+    };
     int l = 1;
-    while (l < nlev && L_[l].n > DENSE_TAIL_MAX) ++l;
+    while (l < nlev && !fits(l)) ++l;
     if (l >= nlev) return;
     for (int k = l; k < nlev; ++k)
       if (L_[k].ml_cycle == KCYCLE || L_[k].ml_cycle == KCYCLESYM) return;
     DLevel<V>& D = L_[l];
     if (l == nlev - 1 && (D.sm.solver == DENSE_LU || D.sm.smoother == NOPREC)) return;
-    const int n = D.n;
-    V* B = ar_.alloc<V>((size_t)n * n);
-    for (int j = 0; j < n; ++j) {
-      unit_vec_kernel<V><<<nblk(n), BS, 0, s_>>>(n, D.x2l, j);
-      int rc = inner_ml_aply(l, 'N');
-      if (rc) return;  // the cycle stays as it is
-      col_store_kernel<V><<<nblk(n), BS, 0, s_>>>(n, D.y2l, B, j);
+    const int n = D.n, ld = (n + 63) / 64 * 64;
+    DevArena tmp;
+    std::vector<tail::Lev> T(nlev - l);
+    auto smoother = [&](const SmootherData& h, const DSmoother<V>& d) {
+      tail::Sm t;
+      t.smoother = h.smoother;
+      t.solver = h.solver;
+      t.nnz_nd = h.nnz_nd;
+      t.dinv = d.dinv;
+      if (h.smoother == NOPREC) return t;
+      if (h.nnz_nd > 0) t.nd = make_src(h.nd, tmp, s_);
+      if (!h.dv.empty()) t.dv = tmp.upload(h.dv.data(), h.dv.size(), s_);
+      if (h.solver == ILU_N || h.solver == GS || h.solver == BWGS) {
+        t.l = make_src(h.l, tmp, s_);
+        t.u = make_src(h.u, tmp, s_);
+        t.lptr = d.lptr_d;
+        t.lrows = d.lrows;
+        t.nl = (int)d.lptr.size() - 1;
+        t.uptr = d.uptr_d;
+        t.urows = d.urows;
+        t.nu = (int)d.uptr.size() - 1;
+      }
+      return t;
+    };
+    for (int k = l; k < nlev; ++k) {
+      const Level& H = hprec_->precv[k];
+      tail::Lev& t = T[k - l];
+      t.n = L_[k].n;
+      t.pre = L_[k].sweeps_pre;
+      t.post = L_[k].sweeps_post;
+      t.cycle = L_[k].ml_cycle;
+      t.a = make_src(H.a, tmp, s_);
+      if (k > l) {
+        t.p = make_src(H.p, tmp, s_);
+        t.r = make_src(H.r, tmp, s_);
+      }
+      // the products of a level go down from it: its own R and P are the next
+      // level's
+      t.sm = smoother(H.smd, L_[k].sm);
+      t.has2 = L_[k].has_sm2;
+      if (t.has2) t.sm2 = smoother(H.smd2, L_[k].sm2);
+      double* w = tmp.alloc<double>(5 * (size_t)t.n * ld);
+      for (double** v : {&t.x, &t.y, &t.ty, &t.tx, &t.t1}) {
+        *v = w;
+        w += (size_t)t.n * ld;
+      }
     }
+    tail::Cycle cyc(T, n, ld, s_);
+    if (!cyc.run()) {  // the cycle stays as it is
+      HIPCHECK(hipStreamSynchronize(s_));
+      return;
+    }
+    V* B = ar_.alloc<V>((size_t)n * ld);
+    tail::mstore_kernel<V><<<dim3(n, (ld + 255) / 256), 256, 0, s_>>>(n, ld, T[0].y, ld, B);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s_));
     tail_b_ = B;
+    tail_ld_ = ld;
     tail_lev_ = l;
   }
   // y2l = B x2l at the tail level
   void tail_apply(DLevel<V>& D) {
-    tail_gemv_kernel<V><<<(D.n + BS / 64 - 1) / (BS / 64), BS, 0, s_>>>(D.n, tail_b_, D.x2l, D.y2l);
+    tail_gemv_kernel<V><<<(D.n + BS / 64 - 1) / (BS / 64), BS, 0, s_>>>(D.n, tail_ld_, tail_b_, D.x2l, D.y2l);
     HIPCHECK(hipGetLastError());
   }
 
@@ -637,8 +706,12 @@ class DevPrecT : public DevPrec {
     const bool ilu = (H.solver == ILU_N);
     tp::Packed<V> pl, pu;
     const double* d = H.dv.empty() ? nullptr : H.dv.data();
-    if ((ilu || H.solver == GS) && !tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl)) return;
-    if ((ilu || H.solver == BWGS) && !tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu)) return;
+    // (both factors at once; an exception of the second thread arrives by get())
+    auto second = std::async(ilu ? std::launch::async : std::launch::deferred, [&] {
+      return H.solver == GS || tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu);
+    });
+    const bool okl = H.solver == BWGS || tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl);
+    if (!second.get() || !okl) return;
     std::vector<int> pos(n), idx(n);
     auto up = [&](const tp::Packed<V>& f, typename DSmoother<V>::PackedTri& t) {
       for (int p = 0; p < n; ++p) pos[f.rows[p]] = p;

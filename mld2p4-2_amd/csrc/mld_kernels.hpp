@@ -1312,31 +1312,36 @@ __global__ __launch_bounds__(BS) void dia_colscale_kernel(int nr, int nc, int w,
 }
 
 // ------------------------------------------------- dense tail operator
-// y = B x for a dense row-major n x n operator: one wavefront per row, the
-// lanes over the columns, then a fixed-order reduction across the lanes.
+// y = B x for a dense row-major n x n operator with rows of ld values (a
+// multiple of 64, padding zero): one wavefront per row, every lane 16 bytes of
+// the row at a time and four of those in flight, then a fixed-order reduction
+// across the lanes.  Bound by reading B (from the Infinity Cache up to a few
+// thousand rows).
 template <typename V>
-__global__ __launch_bounds__(BS) void tail_gemv_kernel(int n, const V* __restrict__ B, const V* __restrict__ x,
-                                                       V* __restrict__ y) {
+__global__ __launch_bounds__(BS) void tail_gemv_kernel(int n, int ld, const V* __restrict__ B,
+                                                       const V* __restrict__ x, V* __restrict__ y) {
+  constexpr int W = 16 / (int)sizeof(V);
+  typedef V vec __attribute__((ext_vector_type(W)));
   const int row = blockIdx.x * (BS / 64) + (int)(threadIdx.x / 64);
   const int lane = threadIdx.x % 64;
   if (row >= n) return;  // whole wavefronts
-  const V* b = B + (size_t)row * n;
+  const vec* b = (const vec*)(B + (size_t)row * ld);
+  const int nq = ld / W;  // chunks of a row; x ends at n inside the last ones
   V acc = (V)0;
-  for (int j = lane; j < n; j += 64) acc += b[j] * x[j];
+  for (int q0 = lane; q0 < nq; q0 += 4 * 64) {
+    vec v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = q0 + u * 64 < nq ? b[q0 + u * 64] : (vec)(V)0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = (q0 + u * 64) * W;
+#pragma unroll
+      for (int e = 0; e < W; ++e)
+        if (j + e < n) acc += v[u][e] * x[j + e];
+    }
+  }
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
   if (lane == 0) y[row] = acc;
-}
-// x = e_j
-template <typename V>
-__global__ __launch_bounds__(BS) void unit_vec_kernel(int n, V* __restrict__ x, int j) {
-  const int i = blockIdx.x * BS + threadIdx.x;
-  if (i < n) x[i] = (i == j) ? (V)1 : (V)0;
-}
-// column j of the row-major n x n B = y
-template <typename V>
-__global__ __launch_bounds__(BS) void col_store_kernel(int n, const V* __restrict__ y, V* __restrict__ B, int j) {
-  const int i = blockIdx.x * BS + threadIdx.x;
-  if (i < n) B[(size_t)i * n + j] = y[i];
 }
 // ND D of a SELD operator: val times c at each entry's column (decoded as
 // in seld_kernel), one thread per position
