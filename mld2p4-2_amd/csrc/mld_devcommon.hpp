@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
@@ -57,6 +58,13 @@ struct DMat {
   uint16_t* dja = nullptr;
   int* ja = nullptr;
   V* val = nullptr;
+  // DIA with at most 256 distinct rows: class of each row, the classes'
+  // values, the commonest class (diac_kernel); ctab_d: the table holds the
+  // smoother's d too
+  uint8_t* cls = nullptr;
+  V* ctab = nullptr;
+  DiaClass<V> cdef{};
+  bool ctab_d = false;
 };
 
 template <typename V>
@@ -446,10 +454,84 @@ struct has_pair : std::false_type {};
 template <class E>
 struct has_pair<E, std::void_t<decltype(std::declval<const E&>().aligned2())>> : std::true_type {};
 
+// epilogues that take d_i from the caller
+template <class E, class = void>
+struct has_pair_d : std::false_type {};
+template <class E>
+struct has_pair_d<E, std::void_t<decltype(&E::pair_d)>> : std::true_type {};
+template <class G>
+struct gather_x : std::false_type {};
+template <typename V, typename XT>
+struct gather_x<GatherX<V, XT>> : std::true_type {};
+
+// Row classes of a DIA operator (see diac_kernel), d: the smoother's diagonal
+// (null: not used with it).  Left out below DIACLS_MIN_ROWS rows, where the
+// values stay in the caches.
+constexpr int DIACLS_MIN_ROWS = 32768;
+template <typename V>
+static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
+  m.cls = nullptr;
+  if (m.fmt != FMT_DIA || m.nr < DIACLS_MIN_ROWS || m.w < 1 || (d && m.w > 7)) return;
+  struct Work {  // one allocation; from tab on copied back together
+    unsigned long long keys[DIACLS_SLOTS];
+    int rep[DIACLS_SLOTS], num[DIACLS_SLOTS];
+    V tab[8 * 256];
+    int many, at[DIACLS_NS];
+  };
+  DevArena tmp;
+  Work* w = tmp.alloc<Work>(1);
+  HIPCHECK(hipMemsetAsync(w, 0, sizeof(Work), s));
+  dia_class_keys<V><<<nblk(m.nr), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep, &w->many);
+  HIPCHECK(hipGetLastError());
+  int n = 0;
+  HIPCHECK(hipMemcpyAsync(&n, &w->many, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIPCHECK(hipStreamSynchronize(s));
+  if (n > 256) return;
+  uint8_t* cls = ar.alloc<uint8_t>((size_t)m.nr);
+  dia_class_number<V><<<1, BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep, w->num, w->tab);
+  dia_class_rows<V><<<nblk(m.nr), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->num, w->tab, cls, &w->many);
+  dia_class_sample<<<1, DIACLS_NS, 0, s>>>(m.nr, cls, w->at);
+  HIPCHECK(hipGetLastError());
+  Work host;
+  const size_t skip = offsetof(Work, tab);
+  HIPCHECK(hipMemcpyAsync((char*)&host + skip, (char*)w + skip, sizeof(Work) - skip, hipMemcpyDeviceToHost, s));
+  HIPCHECK(hipStreamSynchronize(s));
+  if (host.many > 256) return;
+  // the commonest class: the majority of the sampled rows
+  int count[256] = {}, best = host.at[0];
+  for (int q = 0; q < DIACLS_NS; ++q)
+    if (++count[host.at[q]] > count[best]) best = host.at[q];
+  m.ctab = ar.alloc<V>(8 * 256);
+  HIPCHECK(hipMemcpyAsync(m.ctab, w->tab, sizeof(host.tab), hipMemcpyDeviceToDevice, s));
+  HIPCHECK(hipStreamSynchronize(s));
+  m.cls = cls;
+  m.ctab_d = d != nullptr;
+  m.cdef.c = best;
+  m.cdef.n = n;
+  for (int k = 0; k < 8; ++k) m.cdef.v[k] = host.tab[8 * best + k];
+  if (std::getenv("MLD_VERBOSE"))
+    std::fprintf(stderr, "[mld] %d x %d operator (DIA): %d distinct rows\n", m.nr, m.nc, n);
+}
+
 // DIA launch (with its final reduction when K > 0): two adjacent rows per
 // thread when the epilogue has the two-row form and the arrays allow it.
 template <int K, typename C, typename V, class G, class E>
 static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
+  if constexpr (gather_x<G>::value && has_pair<E>::value) {
+    if (m.cls && e.aligned2() && (!has_pair_d<E>::value || m.ctab_d)) {
+      constexpr bool D = has_pair_d<E>::value;
+      constexpr int RPB = 2 * DIACLS_P * BS;
+      const int nbp = (int)(((int64_t)m.nr + RPB - 1) / RPB);
+      const int xc = xcd_chunk(m.xmap, nbp, RPB);
+      if (m.w == 7)
+        diac_kernel<C, 7, K, D><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.cls, m.ctab, m.cdef, g.x, e, red, xc);
+      else
+        diac_kernel<C, 0, K, D><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.cls, m.ctab, m.cdef, g.x, e, red, xc);
+      if constexpr (K > 0) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nbp, red.partial, red.result);
+      HIPCHECK(hipGetLastError());
+      return;
+    }
+  }
   // (FP64 values only: with FP32 values the two-row form was slower, the
   // fine-level FP32 residual 94 -> 127 us at 256^3, the FP32-stored Krylov
   // product summed in FP64 144 -> 150 us)

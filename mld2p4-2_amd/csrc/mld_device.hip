@@ -49,6 +49,7 @@ class DevPrecT : public DevPrec {
       D.n = H.a.nr;
       double t0 = wall_seconds();
       D.a = upload_tuned<V>(H.a, ar_, s_, p.dev_format);
+      dia_classes<V>(D.a, nullptr, ar_, s_);
       phase_log("upload A", l + 1, wall_seconds() - t0);
       if (l > 0) {
         t0 = wall_seconds();
@@ -91,6 +92,7 @@ class DevPrecT : public DevPrec {
         akry_is32_ = true;
       } else {
         akry_ = upload_mat<double>(p.precv[0].a, ar_, s_, p.dev_format);
+        dia_classes<double>(akry_, nullptr, ar_, s_);
       }
     }
     n0_ = L_[0].n;
@@ -635,6 +637,8 @@ class DevPrecT : public DevPrec {
                                                                                S.dv, S.ndd.val);
       }
       HIPCHECK(hipGetLastError());
+      dia_classes<V>(S.nd, S.dv, ar_, s_);
+      dia_classes<V>(S.ndd, S.dv, ar_, s_);
     }
     if (H.solver == ILU_N || H.solver == GS || H.solver == BWGS) {
       S.l = upload_mat<V>(H.l, ar_, s_, 1, 1);  // CSR (rows summed in stored order)

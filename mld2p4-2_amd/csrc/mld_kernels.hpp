@@ -102,20 +102,25 @@ struct EpiRes {  // r = b - A x     (psb_geaxpby + psb_spmm(-1,A,x,1,r))
   }
   bool aligned2() const { return al2(b, sizeof(BT)) && al2(r, sizeof(V)); }
 };
+// (one_d, pair_d: with d_i from the caller, see diac_kernel)
 template <typename V, typename BT, typename YT, bool ADD, bool NT = false>
 struct EpiJac {  // t = d*(b - ND y);  y = t  or  y = y + t
   const V* __restrict__ d;
   const BT* __restrict__ b;
   YT* __restrict__ y;
-  __device__ __forceinline__ void operator()(int i, V acc, double*) const {
-    V t = d[i] * ((V)b[i] - acc);
+  __device__ __forceinline__ void operator()(int i, V acc, double* dd) const { one_d(i, acc, d[i], dd); }
+  __device__ __forceinline__ void one_d(int i, V acc, V di, double*) const {
+    V t = di * ((V)b[i] - acc);
     if (ADD) stnt<NT>(y + i, (YT)((V)y[i] + t));
     else stnt<NT>(y + i, (YT)t);
   }
-  __device__ __forceinline__ void pair(int i, V a0, V a1, double*) const {
+  __device__ __forceinline__ void pair(int i, V a0, V a1, double* pd) const {
     const vec2_t<V> dd = *(const vec2_t<V>*)(d + i);
+    pair_d(i, a0, a1, dd.x, dd.y, pd);
+  }
+  __device__ __forceinline__ void pair_d(int i, V a0, V a1, V d0, V d1, double*) const {
     const vec2_t<BT> bb = *(const vec2_t<BT>*)(b + i);
-    const V t0 = dd.x * ((V)bb.x - a0), t1 = dd.y * ((V)bb.y - a1);
+    const V t0 = d0 * ((V)bb.x - a0), t1 = d1 * ((V)bb.y - a1);
     if (ADD) {
       const vec2_t<YT> yy = *(const vec2_t<YT>*)(y + i);
       stnt<NT>((vec2_t<YT>*)(y + i), vec2_t<YT>{(YT)((V)yy.x + t0), (YT)((V)yy.y + t1)});
@@ -136,17 +141,22 @@ struct EpiJacOut {
   const V* yin;
   YO* yout;  // FP64 output, or (YO = V) yin itself
   const double* u;
-  __device__ __forceinline__ void operator()(int i, V acc, double* dd) const {
-    const V t = d[i] * ((V)b[i] - acc);
+  __device__ __forceinline__ void operator()(int i, V acc, double* dd) const { one_d(i, acc, d[i], dd); }
+  __device__ __forceinline__ void one_d(int i, V acc, V di, double* dd) const {
+    const V t = di * ((V)b[i] - acc);
     const V yn = yin[i] + t;
     stnt<NT>(yout + i, (YO)yn);
     if (u) dd[0] = u[i] * (double)yn;
   }
   // two rows; their dot terms are added to dd
   __device__ __forceinline__ void pair(int i, V a0, V a1, double* dd) const {
-    const vec2_t<V> dv = *(const vec2_t<V>*)(d + i), yv = *(const vec2_t<V>*)(yin + i);
+    const vec2_t<V> dv = *(const vec2_t<V>*)(d + i);
+    pair_d(i, a0, a1, dv.x, dv.y, dd);
+  }
+  __device__ __forceinline__ void pair_d(int i, V a0, V a1, V d0, V d1, double* dd) const {
+    const vec2_t<V> yv = *(const vec2_t<V>*)(yin + i);
     const vec2_t<BT> bb = *(const vec2_t<BT>*)(b + i);
-    const V y0 = yv.x + dv.x * ((V)bb.x - a0), y1 = yv.y + dv.y * ((V)bb.y - a1);
+    const V y0 = yv.x + d0 * ((V)bb.x - a0), y1 = yv.y + d1 * ((V)bb.y - a1);
     stnt<NT>((vec2_t<YO>*)(yout + i), vec2_t<YO>{(YO)y0, (YO)y1});
     if (u) {
       const vec2_t<double> uu = *(const vec2_t<double>*)(u + i);
@@ -480,6 +490,210 @@ __global__ __launch_bounds__(BS) void dia_kernel(int nr, int nc, int nd, DiaOff 
     }
   }
   if constexpr (K > 0) block_partials<K>(dd, red.partial, lb);
+}
+
+// DIA with row classes: where an operator has at most 256 distinct rows (its
+// values by diagonal, and the smoother's d_i with them), as constant
+// coefficients give, one byte per row names the row's class instead of nd
+// values read per row.  The values of the commonest class arrive as kernel
+// arguments (scalar registers); the others' are in LDS, copied while the
+// vector's loads are in flight.  A thread takes DIACLS_P pairs of adjacent
+// rows, 2 BS rows apart.  Per row the arithmetic of dia_kernel.  Bound by the
+// vectors: the residual at 256^3 FP64 moves 3 n values and n bytes, 420 MB
+// instead of 1.34 GB.  At 256^3, FP64, inside solves: residual 207 -> 82 us
+// (5.1 TB/s), first two sweeps 212 -> 64, last sweeps with the dot 265 -> 100,
+// Krylov product 200 -> 60; one pair per thread and the classes' values from
+// memory: 96, 74, 111, 68; four pairs: 93, 66, 101, 63.
+template <typename S>
+struct DiaClass {
+  S v[8];   // values of the commonest class (7: d where the table holds it)
+  int c;    // its number
+  int n;    // classes
+};
+constexpr int DIACLS_P = 2;
+template <typename C, int ND, int K, bool D, class E, typename S, typename XT>
+__global__ __launch_bounds__(BS) void diac_kernel(int nr, int nc, int nd, DiaOff off,
+                                                   const uint8_t* __restrict__ cls, const S* __restrict__ tab,
+                                                   DiaClass<S> def, const XT* __restrict__ x, E e, Red red,
+                                                   int xchunk) {
+  typedef XT ux2 __attribute__((ext_vector_type(2), aligned(sizeof(XT))));
+  constexpr int P = DIACLS_P, NK = ND > 0 ? ND : 8;
+  __shared__ S lt[8 * 256];
+  const int lb = xcd_block(xchunk);
+  const int b0 = 2 * P * lb * BS;
+  const int ndg = ND > 0 ? ND : nd;
+  XT x0[P][NK], x1[P][NK];
+  int c0[P], c1[P];
+  // (offsets ascend) no row of the block reaches outside: pairs by one load
+  if (b0 + off.o[0] >= 0 && b0 + 2 * P * BS + off.o[ndg - 1] <= nc && b0 + 2 * P * BS <= nr) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int i0 = b0 + 2 * (p * BS + (int)threadIdx.x);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        if (ND == 0 && k >= ndg) break;
+        const ux2 t = *(const ux2*)(x + (i0 + off.o[k]));
+        x0[p][k] = t.x;
+        x1[p][k] = t.y;
+      }
+      const uint16_t cc = *(const uint16_t*)(cls + i0);
+      c0[p] = cc & 0xff;
+      c1[p] = cc >> 8;
+    }
+  } else {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int i0 = min(b0 + 2 * (p * BS + (int)threadIdx.x), nr - 1), i1 = min(i0 + 1, nr - 1);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        if (ND == 0 && k >= ndg) break;
+        x0[p][k] = x[min(max(i0 + off.o[k], 0), nc - 1)];
+        x1[p][k] = x[min(max(i1 + off.o[k], 0), nc - 1)];
+      }
+      c0[p] = cls[i0];
+      c1[p] = cls[i1];
+    }
+  }
+  for (int t = threadIdx.x; t < 8 * def.n; t += BS) lt[t] = tab[t];
+  __syncthreads();
+  double pd[2] = {0.0, 0.0};
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int i0 = b0 + 2 * (p * BS + (int)threadIdx.x);
+    C a0 = 0, a1 = 0, d0 = (C)def.v[7], d1 = (C)def.v[7];
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      if (ND == 0 && k >= ndg) break;
+      a0 = a0 + (C)def.v[k] * (C)x0[p][k];
+      a1 = a1 + (C)def.v[k] * (C)x1[p][k];
+    }
+    if (c0[p] != def.c || c1[p] != def.c) {
+      const S *t0 = lt + 8 * c0[p], *t1 = lt + 8 * c1[p];
+      a0 = 0;
+      a1 = 0;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        if (ND == 0 && k >= ndg) break;
+        a0 = a0 + (C)t0[k] * (C)x0[p][k];
+        a1 = a1 + (C)t1[k] * (C)x1[p][k];
+      }
+      if (D) {
+        d0 = (C)t0[7];
+        d1 = (C)t1[7];
+      }
+    }
+    if (i0 + 1 < nr) {
+      if constexpr (D) e.pair_d(i0, a0, a1, d0, d1, pd);
+      else e.pair(i0, a0, a1, pd);
+    } else if (i0 < nr) {
+      double d1s[2] = {0.0, 0.0};
+      if constexpr (D) e.one_d(i0, a0, d0, d1s);
+      else e(i0, a0, d1s);
+      pd[0] += d1s[0];
+      pd[1] += d1s[1];
+    }
+  }
+  if constexpr (K > 0) block_partials<K>(pd, red.partial, lb);
+}
+
+// Row classes of a DIA operator.  Keys (hashes of a row's bits, never 0) are
+// put into an open table of DIACLS_SLOTS slots; more than 256 of them end the
+// search (many).  The numbers are then given by slot, and every row is compared
+// with the one that stands for its class, so that two rows of one hash are
+// found out (many).
+constexpr int DIACLS_SLOTS = 2048;
+template <typename S>
+__device__ __forceinline__ uint64_t dia_row_key(int nr, int w, const S* __restrict__ val, const S* __restrict__ d,
+                                                int i) {
+  uint64_t h = 0x9e3779b97f4a7c15ull;
+  for (int k = 0; k <= w; ++k) {
+    uint64_t u = 0;
+    if (k == w && !d) break;
+    const S v = k < w ? val[(int64_t)k * nr + i] : d[i];
+    __builtin_memcpy(&u, &v, sizeof(S));
+    h = (h ^ u) * 0xbf58476d1ce4e5b9ull;
+    h ^= h >> 29;
+  }
+  return h | 1;
+}
+template <typename S>
+__global__ __launch_bounds__(BS) void dia_class_keys(int nr, int w, const S* __restrict__ val,
+                                                     const S* __restrict__ d, unsigned long long* keys, int* rep,
+                                                     int* many) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i >= nr || __hip_atomic_load(many, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 256) return;
+  const unsigned long long key = dia_row_key(nr, w, val, d, i);
+  int s = (int)(key >> 20) & (DIACLS_SLOTS - 1);
+  for (int probe = 0; probe < DIACLS_SLOTS; ++probe, s = (s + 1) & (DIACLS_SLOTS - 1)) {
+    unsigned long long q = __hip_atomic_load(keys + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (q == 0) {
+      q = atomicCAS(keys + s, 0ull, key);
+      if (q == 0) {  // this row stands for the class
+        rep[s] = i;
+        atomicAdd(many, 1);
+        return;
+      }
+    }
+    if (q == key || __hip_atomic_load(many, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 256) return;
+  }
+}
+// slots -> numbers, and the table (8 values per class; 7: d); one workgroup
+template <typename S>
+__global__ __launch_bounds__(BS) void dia_class_number(int nr, int w, const S* __restrict__ val,
+                                                       const S* __restrict__ d,
+                                                       const unsigned long long* __restrict__ keys,
+                                                       const int* __restrict__ rep, int* __restrict__ num,
+                                                       S* __restrict__ tab) {
+  __shared__ int count[BS + 1];
+  constexpr int PER = DIACLS_SLOTS / BS;
+  const int t = threadIdx.x;
+  int mine = 0;
+  for (int q = 0; q < PER; ++q) mine += keys[t * PER + q] != 0;
+  count[t + 1] = mine;
+  if (t == 0) count[0] = 0;
+  __syncthreads();
+  if (t == 0)
+    for (int q = 0; q < BS; ++q) count[q + 1] += count[q];
+  __syncthreads();
+  int c = count[t];
+  for (int q = 0; q < PER; ++q) {
+    const int s = t * PER + q;
+    if (keys[s] == 0) continue;
+    num[s] = c;
+    const int i = rep[s];
+    for (int k = 0; k < 8; ++k) tab[8 * c + k] = k < w ? val[(int64_t)k * nr + i] : (k == 7 && d ? d[i] : (S)0);
+    ++c;
+  }
+}
+// classes of DIACLS_NS rows spread over the operator
+constexpr int DIACLS_NS = 64;
+__global__ __launch_bounds__(DIACLS_NS) void dia_class_sample(int nr, const uint8_t* __restrict__ cls,
+                                                              int* __restrict__ at) {
+  at[threadIdx.x] = cls[(int64_t)nr * (2 * threadIdx.x + 1) / (2 * DIACLS_NS)];
+}
+template <typename S>
+__global__ __launch_bounds__(BS) void dia_class_rows(int nr, int w, const S* __restrict__ val,
+                                                     const S* __restrict__ d,
+                                                     const unsigned long long* __restrict__ keys,
+                                                     const int* __restrict__ num, const S* __restrict__ tab,
+                                                     uint8_t* __restrict__ cls, int* many) {
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i >= nr) return;
+  const unsigned long long key = dia_row_key(nr, w, val, d, i);
+  int s = (int)(key >> 20) & (DIACLS_SLOTS - 1);
+  for (int probe = 0; probe < DIACLS_SLOTS && keys[s] != key; ++probe) s = (s + 1) & (DIACLS_SLOTS - 1);
+  const int c = num[s];
+  cls[i] = (uint8_t)c;
+  bool same = keys[s] == key;
+  for (int k = 0; k <= w; ++k) {
+    if (k == w && !d) break;
+    const S v = k < w ? val[(int64_t)k * nr + i] : d[i], t = tab[8 * c + (k < w ? k : 7)];
+    uint64_t p = 0, q = 0;
+    __builtin_memcpy(&p, &v, sizeof(S));
+    __builtin_memcpy(&q, &t, sizeof(S));
+    same = same && p == q;
+  }
+  if (!same) atomicAdd(many, 1000);
 }
 
 // SELL: position p = 64*slice + lane holds row perm[p]; slice s occupies

@@ -24,7 +24,6 @@ def grid2d(nx, ny, nine=False):
     rng = np.random.default_rng(nx * 1000 + ny)
     i = np.arange(n)
     x, y = i % nx, i // nx
-    a = sp.lil_matrix((n, n))
     rows, cols, vals = [], [], []
     for dx in (-1, 0, 1):
         for dy in (-1, 0, 1):
