@@ -208,6 +208,7 @@ static bool host_seld_ok(const HCsr& h) {
   return ok;
 }
 
+constexpr int SELL_FULL_ROWS = 32768;  // rows from which one lane per row occupies the chip
 static FmtChoice choose_format(const HCsr& h, int force) {
   const int maxrow = host_max_row(h);
   const double nnz = (double)h.nnz();
@@ -231,7 +232,12 @@ static FmtChoice choose_format(const HCsr& h, int force) {
     return c;
   }
   if (maxrow <= 16 && (double)h.nr * maxrow <= 1.10 * nnz) { c.fmt = FMT_ELL; return c; }
-  if (h.nr >= 4096) { c.fmt = FMT_SELL; return c; }
+  // SELL, one lane per row, from 4096 rows on, but several lanes per row (CSR)
+  // for rows of 8 entries or more while one lane each leaves most of the chip
+  // without a wavefront and makes a long chain of each row: 6251 rows of 62
+  // entries FP32 13.2 -> 4.6 us, of 215 entries (a restriction) 52 -> 6.9
+  // us; 7809 rows of 29 entries FP64 7.6-11 -> 3.7 us
+  if (h.nr >= 4096 && !(avg >= 8.0 && h.nr < SELL_FULL_ROWS)) { c.fmt = FMT_SELL; return c; }
   return c;
 }
 
