@@ -460,6 +460,18 @@ struct has_pair : std::false_type {};
 template <class E>
 struct has_pair<E, std::void_t<decltype(std::declval<const E&>().aligned2())>> : std::true_type {};
 
+// The end of a reduction over nb blocks: in the kernel itself (red_fuse left
+// the ticket), or by finalize_kernel.
+static inline void red_fuse(Red& red, int nb) {
+  if (nb > RED_FUSE_MAX) red.ticket = nullptr;
+}
+template <int K>
+static void red_finish(const Red& red, int nb, hipStream_t s) {
+  if constexpr (K > 0)
+    if (!red.ticket) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nb, red.partial, red.result);
+  HIPCHECK(hipGetLastError());
+}
+
 // epilogues that take d_i from the caller
 template <class E, class = void>
 struct has_pair_d : std::false_type {};
@@ -529,12 +541,12 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
       constexpr int RPB = 2 * DIACLS_P * BS;
       const int nbp = (int)(((int64_t)m.nr + RPB - 1) / RPB);
       const int xc = xcd_chunk(m.xmap, nbp, RPB);
+      red_fuse(red, nbp);
       if (m.w == 7)
         diac_kernel<C, 7, K, D><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.cls, m.ctab, m.cdef, g.x, e, red, xc);
       else
         diac_kernel<C, 0, K, D><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.cls, m.ctab, m.cdef, g.x, e, red, xc);
-      if constexpr (K > 0) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nbp, red.partial, red.result);
-      HIPCHECK(hipGetLastError());
+      red_finish<K>(red, nbp, s);
       return;
     }
   }
@@ -545,26 +557,26 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
     if ((m.nr & 1) == 0 && al2(m.val, sizeof(V)) && e.aligned2()) {
       const int nbp = (int)(((int64_t)m.nr / 2 + BS - 1) / BS);
       const int xc = xcd_chunk(m.xmap, nbp, 2 * BS);
+      red_fuse(red, nbp);
       if (m.w == 7)
         dia_kernel<C, 7, K, 1, G, E, V, true><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
       else
         dia_kernel<C, 0, K, 1, G, E, V, true><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
-      if constexpr (K > 0) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nbp, red.partial, red.result);
-      HIPCHECK(hipGetLastError());
+      red_finish<K>(red, nbp, s);
       return;
     }
   }
   constexpr int RPT = dia_rpt<K>();
   const int nb = (int)(((int64_t)m.nr + BS * RPT - 1) / (BS * RPT));
   const int xc = xcd_chunk(m.xmap, nb, BS * RPT);
+  red_fuse(red, nb);
   if (m.w == 7) dia_kernel<C, 7, K, RPT><<<nb, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
   else dia_kernel<C, 0, K, RPT><<<nb, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
-  if constexpr (K > 0) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nb, red.partial, red.result);
-  HIPCHECK(hipGetLastError());
+  red_finish<K>(red, nb, s);
 }
 
 template <int K = 0, typename CT = void, typename V, class G, class E>
-static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red{nullptr, nullptr}) {
+static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red{nullptr, nullptr, nullptr}) {
   using C = typename std::conditional<std::is_void<CT>::value, V, CT>::type;
   if (m.nr == 0) return;
   if (m.fmt == FMT_DIA) {
@@ -578,6 +590,7 @@ static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red
     return;
   }
   const int nb = spmv_blocks(m);
+  red_fuse(red, nb);
   if (m.fmt == FMT_ELL) {
     const int xc = xcd_chunk(m.xmap, nb, BS);
     switch (m.w) {
@@ -603,8 +616,7 @@ static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red
       default: csr_launch_l<64, K, C>(m, nb, g, e, s, red); break;
     }
   }
-  if constexpr (K > 0) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nb, red.partial, red.result);
-  HIPCHECK(hipGetLastError());
+  red_finish<K>(red, nb, s);
 }
 
 // True when every value of h is exactly representable in FP32 (then an

@@ -108,6 +108,8 @@ class DevPrecT : public DevPrec {
       nbmax = std::max(nbmax, nblk(n0_));
       partial_ = ar_.alloc<double>(2 * (size_t)nbmax + 64);
     }
+    ticket_ = ar_.alloc<int>(RED_TICKETS);
+    HIPCHECK(hipMemsetAsync(ticket_, 0, RED_TICKETS * sizeof(int), s_));
     scal_ = ar_.alloc<double>(S_NSCAL);
     HIPCHECK(hipMemsetAsync(scal_, 0, S_NSCAL * sizeof(double), s_));
     HIPCHECK(hipHostMalloc((void**)&hscal_, S_NSCAL * sizeof(double), hipHostMallocDefault));
@@ -307,7 +309,7 @@ class DevPrecT : public DevPrec {
     *z = L_[0].y2l;
     if (dot_u && !out_done_) {
       dot_kernel<double, 1, V><<<red_blocks(n0_), BS, 0, s_>>>(n0_, dot_u, L_[0].y2l, nullptr, nullptr,
-                                                               red(dot_slot));
+                                                               red_for(dot_slot, red_blocks(n0_)));
       finalize(1, dot_slot);
       HIPCHECK(hipGetLastError());
     }
@@ -563,17 +565,26 @@ class DevPrecT : public DevPrec {
   DMat<double> akry_t_;  // FP64 A^T for adjoint solves, uploaded on first use
   // Krylov product with A ('N') or A^T ('T'), FP64 arithmetic
   template <int K, class G, class E>
-  void kspmv(char trans, G g, E e, Red r = Red{nullptr, nullptr}) {
+  void kspmv(char trans, G g, E e, Red r = Red{nullptr, nullptr, nullptr}) {
     if (trans == 'T') spmv_launch<K>(akry_t_, g, e, s_, r);
     else if (akry_is32_) spmv_launch<K, double>(akry32_, g, e, s_, r);
     else spmv_launch<K>(akry_, g, e, s_, r);
   }
   bool akry_t_set_ = false;
   double* partial_ = nullptr;
-  Red red(int slot) { return Red{partial_, scal_ + slot}; }
-  // one-block sum of the partials of a streaming reduction over n0_ entries
+  Red red(int slot) { return Red{partial_, scal_ + slot, ticket_}; }
+  // of a kernel of nb blocks launched here: without the ticket where they are many
+  Red red_for(int slot, int nb) {
+    Red r = red(slot);
+    red_fuse(r, nb);
+    return r;
+  }
+  int* ticket_ = nullptr;  // see block_partials
+  // one-block sum of the partials of a streaming reduction over n0_ entries,
+  // launched with red_for
   void finalize(int K, int slot, int nb = -1) {
     if (nb < 0) nb = red_blocks(n0_);
+    if (nb <= RED_FUSE_MAX) return;  // the kernel did it (red_for)
     if (K == 1) finalize_kernel<1><<<1, FIN_T, 0, s_>>>(nb, partial_, scal_ + slot);
     else finalize_kernel<2><<<1, FIN_T, 0, s_>>>(nb, partial_, scal_ + slot);
     HIPCHECK(hipGetLastError());
@@ -1279,7 +1290,7 @@ class DevPrecT : public DevPrec {
   }
   template <bool FIRST, bool ADD>
   void jac_sweep(DLevel<V>& D, DSmoother<V>& S, const V* b, const V* yin, V* yout, char trans) {
-    jac_launch<FIRST, 0>(D, S, b, yin, EpiJac<V, V, V, ADD>{S.dv, b, yout}, trans, Red{nullptr, nullptr});
+    jac_launch<FIRST, 0>(D, S, b, yin, EpiJac<V, V, V, ADD>{S.dv, b, yout}, trans, Red{nullptr, nullptr, nullptr});
   }
   // Last post-smoothing sweep of the fine level (beta = 1): writes the
   // FP64 output of the cycle (or, keeping the FP32 result, y2l itself) and
@@ -1288,7 +1299,7 @@ class DevPrecT : public DevPrec {
   void jac_sweep_out(DLevel<V>& D, DSmoother<V>& S, const V* b, const V* yin, V* y2l, char trans) {
     auto run = [&](auto e) {
       if (dot_u_) jac_launch<FIRST, 1>(D, S, b, yin, e, trans, red(dot_slot_));
-      else jac_launch<FIRST, 0>(D, S, b, yin, e, trans, Red{nullptr, nullptr});
+      else jac_launch<FIRST, 0>(D, S, b, yin, e, trans, Red{nullptr, nullptr, nullptr});
     };
     if (keep32_) run(EpiJacOut<V, V, false, V>{S.dv, b, y2l, y2l, dot_u_});
     else run(EpiJacOut<V, V>{S.dv, b, y2l, out64_, dot_u_});
@@ -1314,13 +1325,14 @@ class DevPrecT : public DevPrec {
       if (fo) {  // y = y + d*x, written as the FP64 output (or in place)
         const int nb = nblk(n);
         if (dot_u_) {
-          if (keep32_) vmul_out_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, dot_u_, red(dot_slot_));
-          else vmul_out_kernel<V, 1><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, dot_u_, red(dot_slot_));
-          finalize_kernel<1><<<1, FIN_T, 0, s_>>>(nb, partial_, scal_ + dot_slot_);
+          const Red rd = red_for(dot_slot_, nb);
+          if (keep32_) vmul_out_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, dot_u_, rd);
+          else vmul_out_kernel<V, 1><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, dot_u_, rd);
+          red_finish<1>(rd, nb, s_);
         } else if (keep32_) {
-          vmul_out_kernel<V, 0, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, nullptr, Red{nullptr, nullptr});
+          vmul_out_kernel<V, 0, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, nullptr, Red{nullptr, nullptr, nullptr});
         } else {
-          vmul_out_kernel<V, 0><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, nullptr, Red{nullptr, nullptr});
+          vmul_out_kernel<V, 0><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, nullptr, Red{nullptr, nullptr, nullptr});
         }
         HIPCHECK(hipGetLastError());
         out_done_ = true;
@@ -1487,8 +1499,8 @@ class DevPrecT : public DevPrec {
   // dot products of level vectors (one or two pairs) into scalar slots
   void ldot(int n, const V* a, const V* b, const V* c, const V* d, int slot) {
     const int nb = red_blocks(n);
-    if (c) dot_kernel<V, 2, V><<<nb, BS, 0, s_>>>(n, a, b, c, d, red(slot));
-    else dot_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, a, b, nullptr, nullptr, red(slot));
+    if (c) dot_kernel<V, 2, V><<<nb, BS, 0, s_>>>(n, a, b, c, d, red_for(slot, nb));
+    else dot_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, a, b, nullptr, nullptr, red_for(slot, nb));
     finalize(c ? 2 : 1, slot, nb);
   }
 
@@ -1609,7 +1621,8 @@ class DevPrecT : public DevPrec {
       throw DevError("sync-free triangular solve: a dependency wait exceeded its bound; results are invalid");
   }
   void dot1(const double* a, const double* b, int slot) {
-    dot_kernel<double, 1, double><<<red_blocks(n0_), BS, 0, s_>>>(n0_, a, b, nullptr, nullptr, red(slot));
+    dot_kernel<double, 1, double><<<red_blocks(n0_), BS, 0, s_>>>(n0_, a, b, nullptr, nullptr,
+                                                                   red_for(slot, red_blocks(n0_)));
     finalize(1, slot);
     HIPCHECK(hipGetLastError());
   }
@@ -1700,7 +1713,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
         cg_pupdate<<<nblk(n), BS, 0, s_>>>(n, (const double*)z, p, scal_, it, x, xnum, xden);
       }
       kspmv<1>(trans, GatherX<double, double>{p}, EpiSetDot<double>{q, p, nullptr}, red(S_SIGMA));
-      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, rs, S_SIGMA, red(S_RR), r32);
+      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, rs, S_SIGMA, red_for(S_RR, nbd), r32);
       xnum = rs;
       xden = S_SIGMA;
       preconv_ = r32 ? r : nullptr;
@@ -1731,7 +1744,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
       }
       // q = A p with p.q (S_DELTA) and p.r (S_DPR) in one pass
       kspmv<2>(trans, GatherX<double, double>{p}, EpiSetDotUW<double>{q, p, r}, red(S_DELTA));
-      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, S_DPR, S_DELTA, red(S_RR), r32);
+      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, S_DPR, S_DELTA, red_for(S_RR, nbd), r32);
       xnum = S_DPR;
       xden = S_DELTA;
       preconv_ = r32 ? r : nullptr;
