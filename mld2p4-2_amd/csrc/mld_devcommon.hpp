@@ -468,7 +468,7 @@ static inline void red_fuse(Red& red, int nb) {
 template <int K>
 static void red_finish(const Red& red, int nb, hipStream_t s) {
   if constexpr (K > 0)
-    if (!red.ticket) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nb, red.partial, red.result);
+    if (!red.ticket) finalize_kernel<K><<<1, FIN_T, 0, s>>>(nb, red);
   HIPCHECK(hipGetLastError());
 }
 
@@ -576,7 +576,7 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
 }
 
 template <int K = 0, typename CT = void, typename V, class G, class E>
-static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red{nullptr, nullptr, nullptr}) {
+static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red{}) {
   using C = typename std::conditional<std::is_void<CT>::value, V, CT>::type;
   if (m.nr == 0) return;
   if (m.fmt == FMT_DIA) {

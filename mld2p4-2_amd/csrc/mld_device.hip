@@ -112,7 +112,8 @@ class DevPrecT : public DevPrec {
     HIPCHECK(hipMemsetAsync(ticket_, 0, RED_TICKETS * sizeof(int), s_));
     scal_ = ar_.alloc<double>(S_NSCAL);
     HIPCHECK(hipMemsetAsync(scal_, 0, S_NSCAL * sizeof(double), s_));
-    HIPCHECK(hipHostMalloc((void**)&hscal_, S_NSCAL * sizeof(double), hipHostMallocDefault));
+    HIPCHECK(hipHostMalloc((void**)&hscal_, (S_NSCAL + 1) * sizeof(double), hipHostMallocCoherent));
+    std::memset(hscal_, 0, (S_NSCAL + 1) * sizeof(double));
     HIPCHECK(hipStreamSynchronize(s_));
     hprec_ = &p;
     const double tt = wall_seconds();
@@ -308,10 +309,9 @@ class DevPrecT : public DevPrec {
     if (rc) return rc;
     *z = L_[0].y2l;
     if (dot_u && !out_done_) {
-      dot_kernel<double, 1, V><<<red_blocks(n0_), BS, 0, s_>>>(n0_, dot_u, L_[0].y2l, nullptr, nullptr,
-                                                               red_for(dot_slot, red_blocks(n0_)));
-      finalize(1, dot_slot);
-      HIPCHECK(hipGetLastError());
+      const Red rd = red_for(dot_slot, red_blocks(n0_));
+      dot_kernel<double, 1, V><<<red_blocks(n0_), BS, 0, s_>>>(n0_, dot_u, L_[0].y2l, nullptr, nullptr, rd);
+      red_finish<1>(rd, red_blocks(n0_), s_);
     }
     return 0;
   }
@@ -565,30 +565,32 @@ class DevPrecT : public DevPrec {
   DMat<double> akry_t_;  // FP64 A^T for adjoint solves, uploaded on first use
   // Krylov product with A ('N') or A^T ('T'), FP64 arithmetic
   template <int K, class G, class E>
-  void kspmv(char trans, G g, E e, Red r = Red{nullptr, nullptr, nullptr}) {
+  void kspmv(char trans, G g, E e, Red r = Red{}) {
     if (trans == 'T') spmv_launch<K>(akry_t_, g, e, s_, r);
     else if (akry_is32_) spmv_launch<K, double>(akry32_, g, e, s_, r);
     else spmv_launch<K>(akry_, g, e, s_, r);
   }
   bool akry_t_set_ = false;
   double* partial_ = nullptr;
-  Red red(int slot) { return Red{partial_, scal_ + slot, ticket_}; }
-  // of a kernel of nb blocks launched here: without the ticket where they are many
-  Red red_for(int slot, int nb) {
-    Red r = red(slot);
+  // reduction into slot; publish: its end also sends every slot to the host,
+  // which waits for them in read_scal
+  Red red(int slot, bool publish = false) {
+    Red r{partial_, scal_ + slot, ticket_, scal_, nullptr, 0};
+    if (publish) {
+      r.host = hscal_;
+      r.seq = ++seq_;
+    }
+    return r;
+  }
+  // of a kernel of nb blocks launched here: without the ticket where they are
+  // many (red_finish then adds the partial sums)
+  Red red_for(int slot, int nb, bool publish = false) {
+    Red r = red(slot, publish);
     red_fuse(r, nb);
     return r;
   }
   int* ticket_ = nullptr;  // see block_partials
-  // one-block sum of the partials of a streaming reduction over n0_ entries,
-  // launched with red_for
-  void finalize(int K, int slot, int nb = -1) {
-    if (nb < 0) nb = red_blocks(n0_);
-    if (nb <= RED_FUSE_MAX) return;  // the kernel did it (red_for)
-    if (K == 1) finalize_kernel<1><<<1, FIN_T, 0, s_>>>(nb, partial_, scal_ + slot);
-    else finalize_kernel<2><<<1, FIN_T, 0, s_>>>(nb, partial_, scal_ + slot);
-    HIPCHECK(hipGetLastError());
-  }
+  unsigned long long seq_ = 0;
   double* scal_ = nullptr;
   double* hscal_ = nullptr;
   const Prec* hprec_ = nullptr;
@@ -1290,7 +1292,7 @@ class DevPrecT : public DevPrec {
   }
   template <bool FIRST, bool ADD>
   void jac_sweep(DLevel<V>& D, DSmoother<V>& S, const V* b, const V* yin, V* yout, char trans) {
-    jac_launch<FIRST, 0>(D, S, b, yin, EpiJac<V, V, V, ADD>{S.dv, b, yout}, trans, Red{nullptr, nullptr, nullptr});
+    jac_launch<FIRST, 0>(D, S, b, yin, EpiJac<V, V, V, ADD>{S.dv, b, yout}, trans, Red{});
   }
   // Last post-smoothing sweep of the fine level (beta = 1): writes the
   // FP64 output of the cycle (or, keeping the FP32 result, y2l itself) and
@@ -1299,7 +1301,7 @@ class DevPrecT : public DevPrec {
   void jac_sweep_out(DLevel<V>& D, DSmoother<V>& S, const V* b, const V* yin, V* y2l, char trans) {
     auto run = [&](auto e) {
       if (dot_u_) jac_launch<FIRST, 1>(D, S, b, yin, e, trans, red(dot_slot_));
-      else jac_launch<FIRST, 0>(D, S, b, yin, e, trans, Red{nullptr, nullptr, nullptr});
+      else jac_launch<FIRST, 0>(D, S, b, yin, e, trans, Red{});
     };
     if (keep32_) run(EpiJacOut<V, V, false, V>{S.dv, b, y2l, y2l, dot_u_});
     else run(EpiJacOut<V, V>{S.dv, b, y2l, out64_, dot_u_});
@@ -1330,9 +1332,9 @@ class DevPrecT : public DevPrec {
           else vmul_out_kernel<V, 1><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, dot_u_, rd);
           red_finish<1>(rd, nb, s_);
         } else if (keep32_) {
-          vmul_out_kernel<V, 0, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, nullptr, Red{nullptr, nullptr, nullptr});
+          vmul_out_kernel<V, 0, V><<<nb, BS, 0, s_>>>(n, S.dv, x, y, y, nullptr, Red{});
         } else {
-          vmul_out_kernel<V, 0><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, nullptr, Red{nullptr, nullptr, nullptr});
+          vmul_out_kernel<V, 0><<<nb, BS, 0, s_>>>(n, S.dv, x, y, out64_, nullptr, Red{});
         }
         HIPCHECK(hipGetLastError());
         out_done_ = true;
@@ -1461,14 +1463,14 @@ class DevPrecT : public DevPrec {
     ldot(n, w, w, nullptr, nullptr, S_K0);  // delta0^2
     add_kernel<V, V, false><<<nb, BS, 0, s_>>>(n, D.y2l, d0);
     spmv_launch(D.a, GatherX<V, V>{d0}, EpiSet<V, V>{v}, s_);
-    if (fcg) ldot(n, d0, w, d0, v, S_K1);  // delta_old, tau
-    else ldot(n, v, w, v, v, S_K1);
+    if (fcg) ldot(n, d0, w, d0, v, S_K1, true);  // delta_old, tau
+    else ldot(n, v, w, v, v, S_K1, true);
     read_scal(S_K0);
     const double delta0 = std::sqrt(hscal_[S_K0]);
     const double delta_old = hscal_[S_K1], tau = hscal_[S_K1 + 1];
     double alpha = delta_old / tau;
     axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)(-alpha), v, (V)1, w);  // w -= alpha v
-    ldot(n, w, w, nullptr, nullptr, S_K0);
+    ldot(n, w, w, nullptr, nullptr, S_K0, true);
     const double l2 = std::sqrt(read_scal(S_K0));
     if (l2 <= 0.25 * delta0) {
       axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)alpha, d0, (V)0, D.y2l);  // y = alpha d0
@@ -1480,10 +1482,10 @@ class DevPrecT : public DevPrec {
       spmv_launch(D.a, GatherX<V, V>{d1}, EpiSet<V, V>{v1}, s_);
       if (fcg) {
         ldot(n, d1, v, d1, v1, S_K1);  // tau1, tau2
-        ldot(n, d1, w, nullptr, nullptr, S_K0);  // tau3
+        ldot(n, d1, w, nullptr, nullptr, S_K0, true);  // tau3
       } else {
         ldot(n, v1, v, v1, v1, S_K1);
-        ldot(n, v1, w, nullptr, nullptr, S_K0);
+        ldot(n, v1, w, nullptr, nullptr, S_K0, true);
       }
       read_scal(S_K0);
       const double tau1 = hscal_[S_K1], tau2 = hscal_[S_K1 + 1], tau3 = hscal_[S_K0];
@@ -1497,11 +1499,16 @@ class DevPrecT : public DevPrec {
     return 0;
   }
   // dot products of level vectors (one or two pairs) into scalar slots
-  void ldot(int n, const V* a, const V* b, const V* c, const V* d, int slot) {
+  void ldot(int n, const V* a, const V* b, const V* c, const V* d, int slot, bool publish = false) {
     const int nb = red_blocks(n);
-    if (c) dot_kernel<V, 2, V><<<nb, BS, 0, s_>>>(n, a, b, c, d, red_for(slot, nb));
-    else dot_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, a, b, nullptr, nullptr, red_for(slot, nb));
-    finalize(c ? 2 : 1, slot, nb);
+    const Red rd = red_for(slot, nb, publish);
+    if (c) {
+      dot_kernel<V, 2, V><<<nb, BS, 0, s_>>>(n, a, b, c, d, rd);
+      red_finish<2>(rd, nb, s_);
+    } else {
+      dot_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, a, b, nullptr, nullptr, rd);
+      red_finish<1>(rd, nb, s_);
+    }
   }
 
   // mld_d_inner_mult (mld_dmlprec_aply.f90:590-809)
@@ -1609,9 +1616,21 @@ class DevPrecT : public DevPrec {
   }
 
  private:
+  // A slot's value after the last published reduction: the host polls the
+  // sequence number behind the slots, and now and then asks whether the
+  // stream has ended or failed instead.
   double read_scal(int slot) {
-    HIPCHECK(hipMemcpyAsync(hscal_, scal_, S_NSCAL * sizeof(double), hipMemcpyDeviceToHost, s_));
-    HIPCHECK(hipStreamSynchronize(s_));
+    const unsigned long long* q = (const unsigned long long*)(hscal_ + S_NSCAL);
+    for (unsigned k = 1; __atomic_load_n(q, __ATOMIC_ACQUIRE) != seq_; ++k) {
+      __builtin_ia32_pause();
+      if (k % 4096 == 0) {
+        const hipError_t e = hipStreamQuery(s_);
+        if (e == hipErrorNotReady) continue;
+        HIPCHECK(e);
+        if (__atomic_load_n(q, __ATOMIC_ACQUIRE) != seq_) throw DevError("a reduction did not report its result");
+        break;
+      }
+    }
     check_abort();
     return hscal_[slot];
   }
@@ -1620,11 +1639,11 @@ class DevPrecT : public DevPrec {
     if (hscal_[S_ABORT] != 0.0)
       throw DevError("sync-free triangular solve: a dependency wait exceeded its bound; results are invalid");
   }
-  void dot1(const double* a, const double* b, int slot) {
-    dot_kernel<double, 1, double><<<red_blocks(n0_), BS, 0, s_>>>(n0_, a, b, nullptr, nullptr,
-                                                                   red_for(slot, red_blocks(n0_)));
-    finalize(1, slot);
-    HIPCHECK(hipGetLastError());
+  void dot1(const double* a, const double* b, int slot, bool publish = false) {
+    const int nb = red_blocks(n0_);
+    const Red rd = red_for(slot, nb, publish);
+    dot_kernel<double, 1, double><<<nb, BS, 0, s_>>>(n0_, a, b, nullptr, nullptr, rd);
+    red_finish<1>(rd, nb, s_);
   }
   void axpby(double a, const double* x, double b, double* y) {
     axpby_kernel<double><<<nblk(n0_), BS, 0, s_>>>(n0_, a, x, b, y);
@@ -1665,10 +1684,8 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
   // bn2 and r = b - A x
   dot1(b, b, S_TMP0);
   kspmv<0>(trans, GatherX<double, double>{x}, EpiRes<double, double>{b, r});
-  dot1(r, r, S_RR);
-  HIPCHECK(hipMemcpyAsync(hscal_, scal_, S_NSCAL * sizeof(double), hipMemcpyDeviceToHost, s_));
-  HIPCHECK(hipStreamSynchronize(s_));
-  check_abort();
+  dot1(r, r, S_RR, true);
+  read_scal(S_RR);
   double bn2 = std::sqrt(hscal_[S_TMP0]);
   if (bn2 == 0.0) bn2 = 1.0;
   *err = std::sqrt(hscal_[S_RR]) / bn2;
@@ -1686,11 +1703,13 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
   struct PreconvReset {
     const double*& p;
     bool& pre0;
+    hipStream_t s;
     ~PreconvReset() {
       p = nullptr;
       pre0 = false;  // a sweep launched ahead for an application that did not follow
+      (void)hipStreamSynchronize(s);  // nor does a cycle launched ahead outlive the call, errors included
     }
-  } preconv_reset{preconv_, pre0_launched_};
+  } preconv_reset{preconv_, pre0_launched_, s_};
   // the deferred solution update x += (num/den) p of the last iteration
   // (slots; -1: none pending), applied by the next direction update or here
   int xnum = -1, xden = -1;
@@ -1698,30 +1717,50 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
     if (xnum >= 0) x_update<<<nblk(n), BS, 0, s_>>>(n, x, p, scal_, xnum, xden);
     xnum = xden = -1;
   };
+  // z (z32 in the FP32 form) = M^-1 r with u.z into slot
+  const V* z32 = nullptr;
+  int rc = 0;
+  auto precondition = [&](const double* u, int slot) {
+    return r32 ? apply_keep32(r, u, slot, &z32) : apply_impl(r, z, trans, u, slot);
+  };
+  // Between the residual's update and its norm's arrival the host enqueues the
+  // next application, so that the GPU does not wait for the host's launches:
+  // all of it where the norm that the last reduction rate leads to is still
+  // above eps, else (also at the first iteration) the fine level's
+  // pre-smoothing alone, so that a solve that ends there has hardly done
+  // anything in vain.  Cycles that read scalars on the host (K) start after
+  // the read.
+  bool ahead = false;
+  double err_prev = 0.0;
+  bool host_cycle = false;
+  for (auto& D : L_) host_cycle |= D.ml_cycle == KCYCLE || D.ml_cycle == KCYCLESYM;
+  auto look_ahead = [&](const double* u, int slot) {
+    ahead = false;
+    if (it >= itmax) return;
+    if (!host_cycle && err_prev > 0.0 && *err * (*err / err_prev) > eps) ahead = precondition(u, slot) == 0;
+    else launch_pre0(r, r32 ? nullptr : z, trans);
+  };
+  auto next_err = [&](double rr) {
+    err_prev = *err;
+    *err = std::sqrt(rr) / bn2;
+  };
   if (method == 0) {  // CG
     while (it < itmax) {
       ++it;
       const int rs = (it & 1) ? S_RHO1 : S_RHO0;
-      if (r32) {  // z = M^-1 r kept in FP32, rho = r.z
-        const V* z32 = nullptr;
-        int rc = apply_keep32(r, r, rs, &z32);
-        if (rc) { flush_x(); return rc; }
-        cg_pupdate<<<nblk(n), BS, 0, s_>>>(n, z32, p, scal_, it, x, xnum, xden);
-      } else {
-        int rc = apply_impl(r, z, trans, r, rs);  // z = M^-1 r, rho = r.z
-        if (rc) { flush_x(); return rc; }
-        cg_pupdate<<<nblk(n), BS, 0, s_>>>(n, (const double*)z, p, scal_, it, x, xnum, xden);
-      }
+      // z = M^-1 r and rho = r.z
+      if (!ahead && (rc = precondition(r, rs))) { flush_x(); return rc; }
+      if (r32) cg_pupdate<<<nblk(n), BS, 0, s_>>>(n, z32, p, scal_, it, x, xnum, xden);
+      else cg_pupdate<<<nblk(n), BS, 0, s_>>>(n, (const double*)z, p, scal_, it, x, xnum, xden);
       kspmv<1>(trans, GatherX<double, double>{p}, EpiSetDot<double>{q, p, nullptr}, red(S_SIGMA));
-      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, rs, S_SIGMA, red_for(S_RR, nbd), r32);
+      const Red rd = red_for(S_RR, nbd, true);
+      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, rs, S_SIGMA, rd, r32);
+      red_finish<1>(rd, nbd, s_);
       xnum = rs;
       xden = S_SIGMA;
       preconv_ = r32 ? r : nullptr;
-      finalize(1, S_RR);
-      HIPCHECK(hipGetLastError());
-      if (it < itmax) launch_pre0(r, r32 ? nullptr : z, trans);
-      read_scal(S_RR);
-      *err = std::sqrt(hscal_[S_RR]) / bn2;
+      look_ahead(r, (it & 1) ? S_RHO0 : S_RHO1);
+      next_err(read_scal(S_RR));
       const double rho_new = hscal_[(it & 1) ? S_RHO1 : S_RHO0], rho_old = hscal_[(it & 1) ? S_RHO0 : S_RHO1];
       if (*err <= eps) break;
       if (hscal_[S_SIGMA] == 0.0 || (it > 1 && rho_old == 0.0) || rho_new == 0.0) break;
@@ -1732,27 +1771,19 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
       ++it;
       // z = M^-1 r and, from the second iteration, gamma = q.z in the same
       // pass (an FP32 preconditioner's z stays in FP32)
-      if (r32) {
-        const V* z32 = nullptr;
-        int rc = apply_keep32(r, it > 1 ? q : nullptr, S_GAMMA, &z32);
-        if (rc) { flush_x(); return rc; }
-        fcg_pupdate<<<nblk(n), BS, 0, s_>>>(n, z32, p, scal_, it, x, xnum, xden);
-      } else {
-        int rc = apply_impl(r, z, trans, it > 1 ? q : nullptr, S_GAMMA);
-        if (rc) { flush_x(); return rc; }
-        fcg_pupdate<<<nblk(n), BS, 0, s_>>>(n, (const double*)z, p, scal_, it, x, xnum, xden);
-      }
+      if (!ahead && (rc = precondition(it > 1 ? q : nullptr, S_GAMMA))) { flush_x(); return rc; }
+      if (r32) fcg_pupdate<<<nblk(n), BS, 0, s_>>>(n, z32, p, scal_, it, x, xnum, xden);
+      else fcg_pupdate<<<nblk(n), BS, 0, s_>>>(n, (const double*)z, p, scal_, it, x, xnum, xden);
       // q = A p with p.q (S_DELTA) and p.r (S_DPR) in one pass
       kspmv<2>(trans, GatherX<double, double>{p}, EpiSetDotUW<double>{q, p, r}, red(S_DELTA));
-      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, S_DPR, S_DELTA, red_for(S_RR, nbd), r32);
+      const Red rd = red_for(S_RR, nbd, true);
+      r_update<<<nbd, BS, 0, s_>>>(n, r, q, scal_, S_DPR, S_DELTA, rd, r32);
+      red_finish<1>(rd, nbd, s_);
       xnum = S_DPR;
       xden = S_DELTA;
       preconv_ = r32 ? r : nullptr;
-      finalize(1, S_RR);
-      HIPCHECK(hipGetLastError());
-      if (it < itmax) launch_pre0(r, r32 ? nullptr : z, trans);
-      read_scal(S_RR);
-      *err = std::sqrt(hscal_[S_RR]) / bn2;
+      look_ahead(q, S_GAMMA);
+      next_err(read_scal(S_RR));
       if (*err <= eps) break;
       if (hscal_[S_DELTA] == 0.0) break;
     }
@@ -1768,7 +1799,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
     double rho_old = 1.0, alpha = 1.0, omega = 1.0;
     while (it < itmax) {
       ++it;
-      dot1(rt, r, S_TMP0);
+      dot1(rt, r, S_TMP0, true);
       const double rho = read_scal(S_TMP0);
       if (rho == 0.0) break;
       if (it == 1) {
@@ -1778,15 +1809,15 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
         axpby(-omega, v, 1.0, p);
         axpby(1.0, r, beta, p);
       }
-      int rc = apply(p, ph, trans);
+      rc = apply(p, ph, trans);
       if (rc) return rc;
-      kspmv<1>(trans, GatherX<double, double>{ph}, EpiSetDot<double>{v, rt, nullptr}, red(S_TMP1));
+      kspmv<1>(trans, GatherX<double, double>{ph}, EpiSetDot<double>{v, rt, nullptr}, red(S_TMP1, true));
       const double rtv = read_scal(S_TMP1);
       if (rtv == 0.0) break;
       alpha = rho / rtv;
       HIPCHECK(hipMemcpyAsync(s, r, n * sizeof(double), hipMemcpyDeviceToDevice, s_));
       axpby(-alpha, v, 1.0, s);
-      dot1(s, s, S_TMP0);
+      dot1(s, s, S_TMP0, true);
       const double sn = std::sqrt(read_scal(S_TMP0)) / bn2;
       if (sn <= eps) {
         axpby(alpha, ph, 1.0, x);
@@ -1796,7 +1827,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
       }
       rc = apply(s, sh, trans);
       if (rc) return rc;
-      kspmv<2>(trans, GatherX<double, double>{sh}, EpiSetDot<double>{t, nullptr, s}, red(S_TMP0));  // t.t, s.t
+      kspmv<2>(trans, GatherX<double, double>{sh}, EpiSetDot<double>{t, nullptr, s}, red(S_TMP0, true));  // t.t, s.t
       read_scal(S_TMP0);
       const double tt = hscal_[S_TMP0], ts = hscal_[S_TMP1];
       omega = (tt == 0.0) ? 0.0 : ts / tt;
@@ -1805,7 +1836,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
       HIPCHECK(hipMemcpyAsync(r, s, n * sizeof(double), hipMemcpyDeviceToDevice, s_));
       axpby(-omega, t, 1.0, r);
       rho_old = rho;
-      dot1(r, r, S_RR);
+      dot1(r, r, S_RR, true);
       *err = std::sqrt(read_scal(S_RR)) / bn2;
       if (*err <= eps) break;
       if (omega == 0.0) break;

@@ -291,7 +291,37 @@ struct Red {  // reduction buffers of a kernel with dot outputs
   double* partial;
   double* result;
   int* ticket;  // RED_TICKETS ints, 0 between launches; null: finalize_kernel follows
+  const double* scal;  // with host: the scalar slots go to host[0..S_NSCAL) when the sums are
+  double* host;        // done, then seq to host[S_NSCAL] (pinned memory; the host waits for it)
+  unsigned long long seq;
 };
+// Scalar slots in device memory.
+enum { S_RHO0 = 0, S_RHO1 = 1, S_SIGMA = 2, S_RR = 3, S_PR = 4, S_GAMMA = 5, S_DELTA = 6, S_DPR = 7,
+       S_TMP0 = 8, S_TMP1 = 9, S_OMEGA = 10, S_ALPHA = 11, S_K0 = 12, S_K1 = 13, S_ABORT = 15, S_NSCAL = 16 };
+// (two-dot reductions write slot and slot + 1: S_DELTA/S_DPR (FCG's p.Ap and
+// p.r), S_TMP0/S_TMP1, S_K1/14; S_ABORT stays clear of them)
+
+// The sums of a reduction, by thread 0's block; with red.host all scalar
+// slots follow into host memory: the copy and the stream synchronisation that
+// reading them took otherwise cost 20-30 us of an idle GPU, the stores 2.
+template <int K>
+__device__ __forceinline__ void put_sums(const double* sum, const Red& red) {
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < K; ++q)
+      __hip_atomic_store(red.result + q, sum[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (!red.host || threadIdx.x >= 64) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (threadIdx.x < S_NSCAL) {
+    const double v = __hip_atomic_load(red.scal + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(red.host + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (threadIdx.x == 0)
+    __hip_atomic_store((unsigned long long*)red.host + S_NSCAL, red.seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // Launches of at most this many blocks add their partial sums themselves.
 // More blocks would wait for one counter (and one workgroup reads 16k partials
 // no faster than finalize_kernel does).
@@ -343,6 +373,7 @@ __device__ __forceinline__ void block_partials(const double* v, const Red& red, 
   }
   __syncthreads();
   if (!last) return;
+  double acc[K];
 #pragma unroll
   for (int q = 0; q < K; ++q) {
     const double* pp = red.partial + (size_t)q * nb;
@@ -352,12 +383,12 @@ __device__ __forceinline__ void block_partials(const double* v, const Red& red, 
       const int b = (int)threadIdx.x + u * BS;
       p[u] = b < nb ? __hip_atomic_load(pp + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
     }
-    double acc = 0.0;
+    acc[q] = 0.0;
 #pragma unroll
-    for (int u = 0; u < RED_FUSE_MAX / BS; ++u) acc += p[u];
-    acc = block_sum(acc, lds);
-    if (threadIdx.x == 0) red.result[q] = acc;
+    for (int u = 0; u < RED_FUSE_MAX / BS; ++u) acc[q] += p[u];
+    acc[q] = block_sum(acc[q], lds);
   }
+  put_sums<K>(acc, red);
 }
 template <int K>
 __device__ __forceinline__ void block_partials(const double* v, const Red& red) {
@@ -370,13 +401,12 @@ __device__ __forceinline__ void block_partials(const double* v, const Red& red) 
 // bound at ~60 us for 64k partials), then a fixed-order wave / block tree.
 constexpr int FIN_T = 1024;
 template <int K>
-__global__ __launch_bounds__(FIN_T) void finalize_kernel(int nb, const double* __restrict__ partial,
-                                                          double* __restrict__ result) {
+__global__ __launch_bounds__(FIN_T) void finalize_kernel(int nb, Red red) {
   __shared__ double lds[K][FIN_T / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
   for (int q = 0; q < K; ++q) {
-    const double* pp = partial + (size_t)q * nb;
+    const double* pp = red.partial + (size_t)q * nb;
     double acc = 0.0;
     int b = threadIdx.x;
     for (; b + 7 * FIN_T < nb; b += 8 * FIN_T) {
@@ -391,12 +421,14 @@ __global__ __launch_bounds__(FIN_T) void finalize_kernel(int nb, const double* _
     if (lane == 0) lds[q][wid] = acc;
   }
   __syncthreads();
-  if ((int)threadIdx.x < K) {
-    double s = 0.0;
+  double sum[K];
 #pragma unroll
-    for (int w = 0; w < FIN_T / 64; ++w) s += lds[threadIdx.x][w];
-    result[threadIdx.x] = s;
+  for (int q = 0; q < K; ++q) {
+    sum[q] = 0.0;
+#pragma unroll
+    for (int w = 0; w < FIN_T / 64; ++w) sum[q] += lds[q][w];
   }
+  put_sums<K>(sum, red);
 }
 
 // Block -> row-block order of a sparse product.  Workgroups reach the 8
@@ -956,12 +988,6 @@ __global__ __launch_bounds__(BS) void dot_kernel(int n, const V* __restrict__ x0
 }
 
 // ------------------------------------------------------------ Krylov steps
-// Scalar slots in device memory.
-enum { S_RHO0 = 0, S_RHO1 = 1, S_SIGMA = 2, S_RR = 3, S_PR = 4, S_GAMMA = 5, S_DELTA = 6, S_DPR = 7,
-       S_TMP0 = 8, S_TMP1 = 9, S_OMEGA = 10, S_ALPHA = 11, S_K0 = 12, S_K1 = 13, S_ABORT = 15, S_NSCAL = 16 };
-// (two-dot reductions write slot and slot + 1: S_DELTA/S_DPR (FCG's p.Ap and
-// p.r), S_TMP0/S_TMP1, S_K1/14; S_ABORT stays clear of them)
-
 // Step length num/den from device slots; 0 when den == 0 (breakdown, detected
 // on the host), which leaves x and r unchanged.
 __device__ __forceinline__ double step_len(const double* __restrict__ scal, int num_slot, int den_slot) {

@@ -49,3 +49,25 @@ def test_dots(eng, n, method):
     assert np.abs(x.cpu().numpy() - xr).max() <= 1e-10 * np.abs(xr).max()
     if n > 16:  # below, the residual is all rounding before the fifth step
         assert it == 5 and abs(err - np.linalg.norm(r) / np.linalg.norm(b)) <= 1e-10
+
+
+@pytest.mark.parametrize("method", ["CG", "FCG"])
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("idim,eps", [(5, 1e-3), (12, 1e-6), (24, 1e-8), (24, 1e-2)])
+def test_ahead(eng, orc, idim, eps, precision, method):
+    """A cycle enqueued before the residual norm is known changes nothing: a
+    solve that stops by its tolerance, by the same number of iterations, and
+    again after both, gives the same bits."""
+    print(f"[ahead] {idim} {eps} {precision} {method}", flush=True)
+    A = orc.gen_pde3d(idim).to_scipy()
+    b = torch.from_numpy(np.random.default_rng(idim).uniform(-1.0, 1.0, A.shape[0])).to("cuda:0")
+    p = eng.MldPrec(device=0).init("ML")
+    for k, v in (("SMOOTHER_TYPE", "L1-JACOBI"), ("AGGR_THRESH", 0.0), ("MIN_COARSE_SIZE", 20)):
+        p.set(k, v)
+    p.set_precision(precision).build(A)
+    x, it, err = eng.psb_krylov(method, A, p, b, eps=eps)
+    assert err <= eps
+    y, jt, e2 = eng.psb_krylov(method, A, p, b, eps=1e-300, itmax=it)
+    assert jt == it and e2 == err and torch.equal(x, y)
+    z, kt, e3 = eng.psb_krylov(method, A, p, b, eps=eps)
+    assert kt == it and e3 == err and torch.equal(x, z)
