@@ -125,7 +125,7 @@ struct DLevel {
   V *x2l = nullptr, *y2l = nullptr, *tx = nullptr, *ty = nullptr, *t1 = nullptr, *t2 = nullptr;
   // K-cycle inner iteration at this level: w, v, v1, d0, d1 (the iterate
   // accumulates in y2l)
-  V *kw = nullptr, *kv = nullptr, *kv1 = nullptr, *kd0 = nullptr, *kd1 = nullptr;
+  V *kv = nullptr, *kv1 = nullptr, *kd0 = nullptr;
   double* wlu = nullptr;
 };
 

@@ -77,8 +77,7 @@ class DevPrecT : public DevPrec {
       if (c != KCYCLE && c != KCYCLESYM) continue;
       DLevel<V>& D = L_[l];
       const size_t n = (size_t)D.n;
-      D.kw = ar_.alloc<V>(n); D.kv = ar_.alloc<V>(n); D.kv1 = ar_.alloc<V>(n);
-      D.kd0 = ar_.alloc<V>(n); D.kd1 = ar_.alloc<V>(n);
+      D.kv = ar_.alloc<V>(n); D.kv1 = ar_.alloc<V>(n); D.kd0 = ar_.alloc<V>(n);
     }
     // Krylov matrix, summed in FP64: level 0's own copy in FP64; in the FP32
     // form, level 0's FP32 copy when every value of A is exact in FP32 (the
@@ -106,6 +105,8 @@ class DevPrecT : public DevPrec {
       nbmax = std::max(nbmax, spmv_blocks(L_[0].sm.nd));
       if (L_[0].has_sm2) nbmax = std::max(nbmax, spmv_blocks(L_[0].sm2.nd));
       nbmax = std::max(nbmax, nblk(n0_));
+      for (auto& D : L_)
+        if (D.kd0) nbmax = std::max(nbmax, spmv_blocks(D.a));
       partial_ = ar_.alloc<double>(2 * (size_t)nbmax + 64);
     }
     ticket_ = ar_.alloc<int>(RED_TICKETS);
@@ -141,9 +142,16 @@ class DevPrecT : public DevPrec {
   // 10 us as one product).
   static constexpr int DENSE_TAIL_MAX = 1024;
   static constexpr double DENSE_TAIL_BYTES = 48e6, DENSE_TAIL_BYTES_TRI = 134.3e6;
+  // Below a K-cycle only the coarsest level's substitutions are one product
+  // (12 unknowns with ILU(0): 20 us in one workgroup, 3 us so; four times a
+  // cycle); the levels above it are not a linear operator, and tail_level()
+  // names none.  Where the transposed cycle is the transposed operator, it
+  // takes the product with tail_bt_ (see build_tail_t).
   int tail_lev_ = -1;
   int tail_ld_ = 0;
+  bool tail_k_ = false;
   V* tail_b_ = nullptr;
+  V* tail_bt_ = nullptr;
   void build_tail() {
     tail_lev_ = -1;
     tail_b_ = nullptr;
@@ -163,10 +171,14 @@ class DevPrecT : public DevPrec {
     int l = 1;
     while (l < nlev && !fits(l)) ++l;
     if (l >= nlev) return;
-    for (int k = l; k < nlev; ++k)
-      if (L_[k].ml_cycle == KCYCLE || L_[k].ml_cycle == KCYCLESYM) return;
+    bool kc = false;
+    for (int k = l; k < nlev; ++k) kc = kc || L_[k].ml_cycle == KCYCLE || L_[k].ml_cycle == KCYCLESYM;
+    tail_k_ = kc;
+    if (kc) l = nlev - 1;  // fits, the levels shrink
+    if (kc && !fits(l)) return;
     DLevel<V>& D = L_[l];
     if (l == nlev - 1 && (D.sm.solver == DENSE_LU || D.sm.smoother == NOPREC)) return;
+    if (kc && D.sm.solver != ILU_N && D.sm.solver != GS && D.sm.solver != BWGS) return;
     const int n = D.n, ld = (n + 63) / 64 * 64;
     DevArena tmp;
     std::vector<tail::Lev> T(nlev - l);
@@ -197,7 +209,7 @@ class DevPrecT : public DevPrec {
       t.n = L_[k].n;
       t.pre = L_[k].sweeps_pre;
       t.post = L_[k].sweeps_post;
-      t.cycle = L_[k].ml_cycle;
+      t.cycle = kc ? VCYCLE : L_[k].ml_cycle;  // (the coarsest level's K-cycle is its smoother)
       t.a = make_src(H.a, tmp, s_);
       if (k > l) {
         t.p = make_src(H.p, tmp, s_);
@@ -227,9 +239,46 @@ class DevPrecT : public DevPrec {
     tail_ld_ = ld;
     tail_lev_ = l;
   }
+  // The transposed cycle below the tail level as one product with B^T: 50 us
+  // of a 72^3 FP32 cycle (six launches, one a substitution in one workgroup)
+  // against 4.  The reference transposes a cycle by exchanging the smoothers,
+  // which is the transposed operator but for a few combinations (an additive
+  // cycle with two smoothers), so the cycle itself decides: it is applied to
+  // one vector without structure and has to agree to the rounding of the value
+  // type, else (also where it refuses 'T') it stays.  Called once the
+  // transposed operators are there.
+  void build_tail_t() {
+    tail_bt_ = nullptr;
+    if (tail_lev_ < 0) return;
+    DLevel<V>& D = L_[tail_lev_];
+    const int n = D.n;
+    std::vector<V> x(n), y(n), z(n);
+    uint64_t h = 0x9e3779b97f4a7c15ull;
+    for (V& v : x) {
+      h = h * 6364136223846793005ull + 1442695040888963407ull;
+      v = (V)((double)(int64_t)h * 0x1p-63);
+    }
+    HIPCHECK(hipMemcpyAsync(D.x2l, x.data(), n * sizeof(V), hipMemcpyHostToDevice, s_));
+    HIPCHECK(hipStreamSynchronize(s_));
+    if (inner_ml_aply(tail_lev_, 'T') != 0) return;
+    HIPCHECK(hipMemcpyAsync(y.data(), D.y2l, n * sizeof(V), hipMemcpyDeviceToHost, s_));
+    V* bt = ar_.alloc<V>((size_t)n * tail_ld_);
+    const dim3 g((tail_ld_ + 31) / 32, (n + 31) / 32);
+    transpose_kernel<V><<<g, dim3(32, 8), 0, s_>>>(n, tail_ld_, tail_b_, bt);
+    tail_gemv(D, bt);
+    HIPCHECK(hipMemcpyAsync(z.data(), D.y2l, n * sizeof(V), hipMemcpyDeviceToHost, s_));
+    HIPCHECK(hipStreamSynchronize(s_));
+    double dmax = 0.0, ymax = 0.0;
+    for (int i = 0; i < n; ++i) {
+      dmax = std::max(dmax, std::fabs((double)y[i] - (double)z[i]));
+      ymax = std::max(ymax, std::fabs((double)y[i]));
+      if (!std::isfinite((double)y[i]) || !std::isfinite((double)z[i])) return;
+    }
+    if (dmax <= (sizeof(V) == 8 ? 1e-13 : 5e-6) * ymax) tail_bt_ = bt;
+  }
   // y2l = B x2l at the tail level
-  void tail_apply(DLevel<V>& D) {
-    tail_gemv_kernel<V><<<(D.n + BS / 64 - 1) / (BS / 64), BS, 0, s_>>>(D.n, tail_ld_, tail_b_, D.x2l, D.y2l);
+  void tail_gemv(DLevel<V>& D, const V* B) {
+    tail_gemv_kernel<V><<<(D.n + BS / 64 - 1) / (BS / 64), BS, 0, s_>>>(D.n, tail_ld_, B, D.x2l, D.y2l);
     HIPCHECK(hipGetLastError());
   }
 
@@ -242,7 +291,7 @@ class DevPrecT : public DevPrec {
   }
 
   size_t device_bytes() const override { return ar_.bytes; }
-  int tail_level() const override { return tail_lev_; }
+  int tail_level() const override { return tail_k_ ? -1 : tail_lev_; }
 
   // y = op(M^-1) x (mld_dprecaply2_vect with alpha = 1, beta = 0).
   int apply(const double* x, double* y, char trans) override { return apply_impl(x, y, trans, nullptr, -1); }
@@ -843,6 +892,7 @@ class DevPrecT : public DevPrec {
       tsm(H.smd, D.sm);
       if (D.has_sm2) tsm(H.smd2, D.sm2);
     }
+    build_tail_t();
     transposes_ = true;
   }
 
@@ -1376,10 +1426,11 @@ class DevPrecT : public DevPrec {
 
   // inner_ml_aply (mld_dmlprec_aply.f90:382-464): dispatch on the level's cycle
   int inner_ml_aply(int level, char trans) {
-    if (level == tail_lev_ && trans == 'N') {
-      tail_apply(L_[level]);
-      return 0;
-    }
+    if (level == tail_lev_)
+      if (const V* B = trans == 'N' ? tail_b_ : tail_bt_) {
+        tail_gemv(L_[level], B);
+        return 0;
+      }
     switch (L_[level].ml_cycle) {
       case ADD_ML: return inner_add(level, trans);
       case MULT_ML: case VCYCLE: case WCYCLE: return inner_mult(level, trans);
@@ -1448,67 +1499,50 @@ class DevPrecT : public DevPrec {
   // reduced on the device and read by the host (the step count and the
   // coefficients are host decisions, as in the reference); the products
   // with A_l are untransposed for 'T' too (:1095, :1137).
+  //
+  // Small levels, so launches and host reads are what it costs: the products
+  // carry their dots, the first step's length and both norms stay on the
+  // device, and one read decides on the second step, whose coefficients the
+  // update kernel forms itself (64^3 under FCG, 12 iterations: 4.4 ms with
+  // every dot, copy and update launched by itself and two reads a step).
   int inneritkcycle(int level, char trans, bool fcg) {
     DLevel<V>& D = L_[level];
     const int n = D.n;
-    const int nb = nblk(n);
-    V *w = D.kw, *v = D.kv, *v1 = D.kv1, *d0 = D.kd0, *d1 = D.kd1;
-    if (!w) return E_UNSUPPORTED;
-    add_kernel<V, V, false><<<nb, BS, 0, s_>>>(n, D.x2l, w);  // w = x2l
-    fill_kernel<V><<<nb, BS, 0, s_>>>(n, D.y2l, (V)0);
+    const int nb = nblk(n), nbr = red_blocks(n);
+    if (!D.kd0) return E_UNSUPPORTED;
+    V *w = D.x2l, *v = D.kv, *v1 = D.kv1;  // the cycle only reads x2l
     int rc = inner_ml_aply(level, trans);
     if (rc) return rc;
     // the scalar slots are shared with the inner iterations of deeper levels,
     // so every dot of this level is formed after its cycle returns
-    ldot(n, w, w, nullptr, nullptr, S_K0);  // delta0^2
-    add_kernel<V, V, false><<<nb, BS, 0, s_>>>(n, D.y2l, d0);
-    spmv_launch(D.a, GatherX<V, V>{d0}, EpiSet<V, V>{v}, s_);
-    if (fcg) ldot(n, d0, w, d0, v, S_K1, true);  // delta_old, tau
-    else ldot(n, v, w, v, v, S_K1, true);
-    read_scal(S_K0);
-    const double delta0 = std::sqrt(hscal_[S_K0]);
-    const double delta_old = hscal_[S_K1], tau = hscal_[S_K1 + 1];
-    double alpha = delta_old / tau;
-    axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)(-alpha), v, (V)1, w);  // w -= alpha v
-    ldot(n, w, w, nullptr, nullptr, S_K0, true);
-    const double l2 = std::sqrt(read_scal(S_K0));
+    std::swap(D.y2l, D.kd0);
+    const V* d0 = D.kd0;
+    // v = A d0, tau and delta_old
+    if (fcg) spmv_launch<2>(D.a, GatherX<V, V>{d0}, EpiSetDotUW<V>{v, d0, w}, s_, red(S_K1));
+    else spmv_launch<2>(D.a, GatherX<V, V>{d0}, EpiSetDot<V>{v, nullptr, w}, s_, red(S_K1));
+    {  // w -= alpha v, ||w||^2 before and after
+      const Red rd = red_for(S_TMP0, nbr, true);
+      kstep_kernel<V><<<nbr, BS, 0, s_>>>(n, w, v, scal_, rd);
+      red_finish<2>(rd, nbr, s_);
+    }
+    const double l2 = std::sqrt(read_scal(S_TMP1)), delta0 = std::sqrt(hscal_[S_TMP0]);
+    const double tau = hscal_[S_K1], alpha = hscal_[S_K1 + 1] / tau;
     if (l2 <= 0.25 * delta0) {
       axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)alpha, d0, (V)0, D.y2l);  // y = alpha d0
     } else {
-      add_kernel<V, V, false><<<nb, BS, 0, s_>>>(n, w, D.x2l);  // x2l = w
       rc = inner_ml_aply(level, trans);
       if (rc) return rc;
-      add_kernel<V, V, false><<<nb, BS, 0, s_>>>(n, D.y2l, d1);
-      spmv_launch(D.a, GatherX<V, V>{d1}, EpiSet<V, V>{v1}, s_);
-      if (fcg) {
-        ldot(n, d1, v, d1, v1, S_K1);  // tau1, tau2
-        ldot(n, d1, w, nullptr, nullptr, S_K0, true);  // tau3
-      } else {
-        ldot(n, v1, v, v1, v1, S_K1);
-        ldot(n, v1, w, nullptr, nullptr, S_K0, true);
-      }
-      read_scal(S_K0);
-      const double tau1 = hscal_[S_K1], tau2 = hscal_[S_K1 + 1], tau3 = hscal_[S_K0];
-      const double tau4 = tau2 - (tau1 * tau1) / tau;
-      alpha = alpha - (tau1 * tau3) / (tau * tau4);
-      const double alpha1 = tau3 / tau4;
-      axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)alpha, d0, (V)0, D.y2l);   // y = alpha d0
-      axpby_kernel<V><<<nb, BS, 0, s_>>>(n, (V)alpha1, d1, (V)1, D.y2l);  // y += alpha1 d1
+      const V* d1 = D.y2l;
+      // v1 = A d1, tau2 and tau3; tau1
+      if (fcg) spmv_launch<2>(D.a, GatherX<V, V>{d1}, EpiSetDotUW<V>{v1, d1, w}, s_, red(S_K1));
+      else spmv_launch<2>(D.a, GatherX<V, V>{d1}, EpiSetDot<V>{v1, nullptr, w}, s_, red(S_K1));
+      const Red rd = red_for(S_K0, nbr);
+      dot_kernel<V, 1, V><<<nbr, BS, 0, s_>>>(n, fcg ? d1 : v1, v, nullptr, nullptr, rd);
+      red_finish<1>(rd, nbr, s_);
+      kcombine_kernel<V><<<nb, BS, 0, s_>>>(n, alpha, tau, scal_, d0, D.y2l);
     }
     HIPCHECK(hipGetLastError());
     return 0;
-  }
-  // dot products of level vectors (one or two pairs) into scalar slots
-  void ldot(int n, const V* a, const V* b, const V* c, const V* d, int slot, bool publish = false) {
-    const int nb = red_blocks(n);
-    const Red rd = red_for(slot, nb, publish);
-    if (c) {
-      dot_kernel<V, 2, V><<<nb, BS, 0, s_>>>(n, a, b, c, d, rd);
-      red_finish<2>(rd, nb, s_);
-    } else {
-      dot_kernel<V, 1, V><<<nb, BS, 0, s_>>>(n, a, b, nullptr, nullptr, rd);
-      red_finish<1>(rd, nb, s_);
-    }
   }
 
   // mld_d_inner_mult (mld_dmlprec_aply.f90:590-809)

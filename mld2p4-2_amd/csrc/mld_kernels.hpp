@@ -1042,6 +1042,39 @@ __global__ __launch_bounds__(BS) void r_update(int n, double* __restrict__ r, co
   block_partials<1>(s, red);
 }
 
+// The K-cycle's first step: w -= alpha v with alpha = delta_old / tau
+// (S_K1 + 1, S_K1); w.w before and after.
+template <typename V>
+__global__ __launch_bounds__(BS) void kstep_kernel(int n, V* __restrict__ w, const V* __restrict__ v,
+                                                   const double* __restrict__ scal, Red red) {
+  const V a = (V)(-(scal[S_K1 + 1] / scal[S_K1]));
+  double s[2] = {0.0, 0.0};
+  const int b = blockIdx.x * BS * RED_EPT + threadIdx.x;
+#pragma unroll
+  for (int e = 0; e < RED_EPT; ++e) {
+    const int i = b + e * BS;
+    if (i < n) {
+      const V w0 = w[i], wi = a * v[i] + w0;
+      w[i] = wi;
+      s[0] += (double)w0 * (double)w0;
+      s[1] += (double)wi * (double)wi;
+    }
+  }
+  block_partials<2>(s, red);
+}
+// Its result after two steps: y = (alpha - tau1 tau3 / (tau tau4)) d0 +
+// (tau3 / tau4) d1, d1 in y; tau1 in S_K0, tau2 and tau3 in S_K1, S_K1 + 1.
+template <typename V>
+__global__ __launch_bounds__(BS) void kcombine_kernel(int n, double alpha, double tau,
+                                                      const double* __restrict__ scal, const V* __restrict__ d0,
+                                                      V* __restrict__ y) {
+  const double tau1 = scal[S_K0], tau2 = scal[S_K1], tau3 = scal[S_K1 + 1];
+  const double tau4 = tau2 - (tau1 * tau1) / tau;
+  const V a = (V)(alpha - (tau1 * tau3) / (tau * tau4)), a1 = (V)(tau3 / tau4);
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i < n) y[i] = a1 * y[i] + a * d0[i];
+}
+
 // x += alpha p (the last deferred update)
 __global__ __launch_bounds__(BS) void x_update(int n, double* __restrict__ x, const double* __restrict__ p,
                                                 const double* __restrict__ scal, int num_slot, int den_slot) {
@@ -1636,6 +1669,19 @@ __global__ __launch_bounds__(BS) void tail_gemv_kernel(int n, int ld, const V* _
   }
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
   if (lane == 0) y[row] = acc;
+}
+// T = B^T, both n x n with rows of ld values (padding zero)
+template <typename V>
+__global__ __launch_bounds__(256) void transpose_kernel(int n, int ld, const V* __restrict__ B, V* __restrict__ T) {
+  __shared__ V t[32][33];
+  const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;  // of T
+  for (int k = threadIdx.y; k < 32; k += 8) {
+    const int r = c0 + k, c = r0 + (int)threadIdx.x;  // of B
+    t[k][threadIdx.x] = r < n && c < ld ? B[(size_t)r * ld + c] : (V)0;
+  }
+  __syncthreads();
+  for (int k = threadIdx.y; k < 32; k += 8)
+    if (r0 + k < n && c0 + (int)threadIdx.x < ld) T[(size_t)(r0 + k) * ld + c0 + threadIdx.x] = t[threadIdx.x][k];
 }
 // ND D of a SELD operator: val times c at each entry's column (decoded as
 // in seld_kernel), one thread per position
