@@ -46,6 +46,7 @@ struct DMat {
   int fmt = FMT_CSR, lanes = 1, w = 0, ld = 0;
   int iters = 0;        // CSR: entries per lane loaded up front (0, 2, 4, 8)
   int rpl = 1;          // block products (32 columns): columns per lane (1, 2, 4)
+  bool longrow = false; // block products: a workgroup per row (bspmm_long_kernel)
   DiaOff off{};         // DIA: diagonal offsets (w diagonals)
   int xmap = 1;         // row-block order: 0 identity, 1 / 3 / 4 chunks of 8192 / 32768 / 131072 rows,
                         // 2 one range per XCD

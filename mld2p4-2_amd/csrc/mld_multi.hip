@@ -298,6 +298,45 @@ __global__ __launch_bounds__(BS) void bdia_kernel(int nr, int nc, int nd, DiaOff
   }
 }
 
+// Y = A X as bspmm_kernel, one workgroup per row: a segment of 8 lanes (4
+// columns each) takes every 32nd entry of the row, and the 32 segments' sums
+// are added pairwise.  For the restrictions and operators of the small levels,
+// where a lane group per row leaves most of the chip idle behind chains of
+// hundreds of gathers (5 workgroups for 40 rows).
+constexpr int BLONG_MAX_ROWS = 4096, BLONG_MIN_ROW = 16;
+template <typename V, class E>
+__global__ __launch_bounds__(BS) void bspmm_long_kernel(const int* __restrict__ irp, const int* __restrict__ ja,
+                                                        const V* __restrict__ val, const V* __restrict__ x, E e) {
+  constexpr int RPL = 4, LPR = MB / RPL, NS = BS / LPR;
+  const int row = blockIdx.x, seg = threadIdx.x / LPR, lane = threadIdx.x % LPR;
+  typedef V vec_t __attribute__((ext_vector_type(RPL)));
+  __shared__ vec_t sh[NS][LPR];
+  const int k1 = irp[row + 1];
+  vec_t acc = (vec_t)(V)0;
+  for (int k = irp[row] + seg; k < k1; k += 4 * NS) {
+    V v[4];
+    vec_t w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int kk = min(k + u * NS, k1 - 1);
+      v[u] = val[kk];
+      w[u] = *reinterpret_cast<const vec_t*>(x + (int64_t)ja[kk] * MB + lane * RPL);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (k + u * NS < k1) acc = acc + v[u] * w[u];
+  }
+  sh[seg][lane] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int h = NS / 2; h >= 1; h >>= 1) {
+    if (seg < h) sh[seg][lane] += sh[seg + h][lane];
+    __syncthreads();
+  }
+  if (threadIdx.x < MB)
+    e(row, (int64_t)row * MB + threadIdx.x, sh[0][threadIdx.x / RPL][threadIdx.x % RPL]);
+}
+
 // y = d_row .* x  (ADD: y += d_row .* x) over n rows of 32 columns
 // Chunk (in blocks) of the row-block order of a block product (see
 // xcd_block).  A row of a 32-column multi-vector is 128 (FP32) or 256 (FP64)
@@ -401,16 +440,16 @@ __device__ __forceinline__ void col_partial(double acc, double* partial) {
   if ((int)threadIdx.x < NB) partial[(int64_t)blockIdx.x * NB + threadIdx.x] = sh[threadIdx.x];
 }
 
-template <int NB>
+template <int NB, typename YT>
 __global__ __launch_bounds__(BS) void mdot_kernel(const int4* __restrict__ bt, const double* __restrict__ x,
-                                                  const double* __restrict__ y, double* __restrict__ partial) {
+                                                  const YT* __restrict__ y, double* __restrict__ partial) {
   constexpr int RPS = BS / NB;
   const int4 b = bt[blockIdx.x];
   const int j = threadIdx.x % NB;
   double acc = 0.0;
   for (int row = b.x + (int)threadIdx.x / NB; row < b.y; row += RPS) {
     const int64_t i = (int64_t)row * NB + j;
-    acc += x[i] * y[i];
+    acc += x[i] * (double)y[i];
   }
   col_partial<NB>(acc, partial);
 }
@@ -442,56 +481,75 @@ __global__ __launch_bounds__(BS) void mfin_kernel(const int* __restrict__ bstart
   if (threadIdx.x == 0) out[c] = sh[0];
 }
 
+// The solution update x += a p of an iteration waits for the next direction
+// update, which reads p anyway (a pass over p fewer per iteration: mcheck_kernel
+// keeps the column's step a, 0 when none is due; mx_kernel applies the last).
+// z in the preconditioner's value type: an FP32 cycle's output is not widened
+// into a vector of its own, 3 x 113 MB less to move for 96^3 x 32 columns.
+// (CG on that: residual and direction updates and both dots 590 us per
+// iteration as separate passes over FP64 vectors.)
+
 // CG direction: p = z (first iteration of the column) or z + (rho/rho_old) p
-template <int NB>
-__global__ __launch_bounds__(BS) void mp_cg_kernel(const int4* __restrict__ bt, const double* __restrict__ z,
-                                                   double* __restrict__ p, const double* __restrict__ rho,
+template <int NB, typename ZT>
+__global__ __launch_bounds__(BS) void mp_cg_kernel(const int4* __restrict__ bt, const ZT* __restrict__ z,
+                                                   double* __restrict__ p, double* __restrict__ x,
+                                                   const double* __restrict__ alpha, const double* __restrict__ rho,
                                                    const double* __restrict__ rho_old, const int* __restrict__ kit,
                                                    const int* __restrict__ done) {
   constexpr int RPS = BS / NB;
   const int4 b = bt[blockIdx.x];
   const int j = threadIdx.x % NB, c = b.z * NB + j;
-  if (done[c]) return;
-  const bool first = (kit[c] == 0);
-  const double beta = first ? 0.0 : rho[c] / rho_old[c];
+  const bool skip = done[c] != 0, first = (kit[c] == 0);
+  const double a = alpha[c];
+  if (skip && a == 0.0) return;
+  const double beta = (first || skip) ? 0.0 : rho[c] / rho_old[c];
   for (int row = b.x + (int)threadIdx.x / NB; row < b.y; row += RPS) {
     const int64_t i = (int64_t)row * NB + j;
-    p[i] = first ? z[i] : z[i] + beta * p[i];
+    if (first) {
+      p[i] = (double)z[i];
+      continue;
+    }
+    const double pi = p[i];
+    if (a != 0.0) x[i] = a * pi + x[i];
+    if (!skip) p[i] = (double)z[i] + beta * pi;
   }
 }
 
 // FCG(1) direction p = z - (gamma/delta_old) p, and sum p.r per column
-template <int NB>
-__global__ __launch_bounds__(BS) void mp_fcg_kernel(const int4* __restrict__ bt, const double* __restrict__ z,
-                                                    double* __restrict__ p, const double* __restrict__ r,
+template <int NB, typename ZT>
+__global__ __launch_bounds__(BS) void mp_fcg_kernel(const int4* __restrict__ bt, const ZT* __restrict__ z,
+                                                    double* __restrict__ p, double* __restrict__ x,
+                                                    const double* __restrict__ alpha, const double* __restrict__ r,
                                                     const double* __restrict__ gamma,
                                                     const double* __restrict__ delta, const int* __restrict__ kit,
                                                     const int* __restrict__ done, double* __restrict__ partial) {
   constexpr int RPS = BS / NB;
   const int4 b = bt[blockIdx.x];
   const int j = threadIdx.x % NB, c = b.z * NB + j;
-  const bool skip = done[c] != 0;
-  const bool first = (kit[c] == 0);
-  const double cf = first ? 0.0 : -(gamma[c] / delta[c]);
+  const bool skip = done[c] != 0, first = (kit[c] == 0);
+  const double a = alpha[c];
+  const double cf = (first || skip) ? 0.0 : -(gamma[c] / delta[c]);
   double acc = 0.0;
-  if (!skip)
+  if (!skip || a != 0.0)
     for (int row = b.x + (int)threadIdx.x / NB; row < b.y; row += RPS) {
       const int64_t i = (int64_t)row * NB + j;
-      const double pi = first ? z[i] : z[i] + cf * p[i];
+      double pi = first ? 0.0 : p[i];
+      if (a != 0.0) x[i] = a * pi + x[i];
+      if (skip) continue;
+      pi = first ? (double)z[i] : (double)z[i] + cf * pi;
       p[i] = pi;
       acc += pi * r[i];
     }
   col_partial<NB>(acc, partial);
 }
 
-// x += a p; r -= a q (a = num/den of the column, 0 when converged or den = 0);
-// sum r.r per column
+// r -= a q (a = num/den of the column, 0 when converged or den = 0); sum r.r
+// per column
 template <int NB>
-__global__ __launch_bounds__(BS) void mxr_kernel(const int4* __restrict__ bt, double* __restrict__ x,
-                                                 double* __restrict__ r, const double* __restrict__ p,
-                                                 const double* __restrict__ q, const double* __restrict__ num,
-                                                 const double* __restrict__ den, const int* __restrict__ done,
-                                                 double* __restrict__ partial, float* __restrict__ r32) {
+__global__ __launch_bounds__(BS) void mr_kernel(const int4* __restrict__ bt, double* __restrict__ r,
+                                                const double* __restrict__ q, const double* __restrict__ num,
+                                                const double* __restrict__ den, const int* __restrict__ done,
+                                                double* __restrict__ partial, float* __restrict__ r32) {
   constexpr int RPS = BS / NB;
   const int4 b = bt[blockIdx.x];
   const int j = threadIdx.x % NB, c = b.z * NB + j;
@@ -500,15 +558,30 @@ __global__ __launch_bounds__(BS) void mxr_kernel(const int4* __restrict__ bt, do
   double acc = 0.0;
   for (int row = b.x + (int)threadIdx.x / NB; row < b.y; row += RPS) {
     const int64_t i = (int64_t)row * NB + j;
+    double ri = r[i];
     if (a != 0.0) {
-      x[i] = a * p[i] + x[i];
-      r[i] = (-a) * q[i] + r[i];
+      ri = (-a) * q[i] + ri;
+      r[i] = ri;
     }
-    const double ri = r[i];
     if (r32) r32[i] = (float)ri;  // FP32 input of the next preconditioner application
     acc += ri * ri;
   }
   col_partial<NB>(acc, partial);
+}
+
+// x += a p, the update that is due when a solve ends
+template <int NB>
+__global__ __launch_bounds__(BS) void mx_kernel(const int4* __restrict__ bt, double* __restrict__ x,
+                                                const double* __restrict__ p, const double* __restrict__ alpha) {
+  constexpr int RPS = BS / NB;
+  const int4 b = bt[blockIdx.x];
+  const int j = threadIdx.x % NB;
+  const double a = alpha[b.z * NB + j];
+  if (a == 0.0) return;
+  for (int row = b.x + (int)threadIdx.x / NB; row < b.y; row += RPS) {
+    const int64_t i = (int64_t)row * NB + j;
+    x[i] = a * p[i] + x[i];
+  }
 }
 
 // Start of a solve: column norms, converged-at-start columns, active count.
@@ -516,10 +589,11 @@ __global__ __launch_bounds__(BS) void mstart_kernel(int ncol, double eps, const 
                                                     const double* __restrict__ rr, double* __restrict__ bn,
                                                     int* __restrict__ kit, int* __restrict__ done,
                                                     int* __restrict__ iters, double* __restrict__ errs,
-                                                    int* __restrict__ active) {
+                                                    double* __restrict__ alpha, int* __restrict__ active) {
   __shared__ double lds[BS / 64];
   double cnt = 0.0;
   for (int c = threadIdx.x; c < ncol; c += BS) {
+    alpha[c] = 0.0;
     double b = std::sqrt(bn2[c]);
     if (b == 0.0) b = 1.0;
     bn[c] = b;
@@ -536,15 +610,20 @@ __global__ __launch_bounds__(BS) void mstart_kernel(int ncol, double eps, const 
 
 // End of an iteration: per-column residual, convergence, breakdown.
 // brk0/brk1: a zero value means breakdown (CG: rho, sigma; FCG: delta).
+// alpha: the step num/den that x still has to take.
 __global__ __launch_bounds__(BS) void mcheck_kernel(int ncol, double eps, int itmax, const double* __restrict__ rr,
                                                     const double* __restrict__ bn, const double* __restrict__ brk0,
                                                     const double* __restrict__ brk1, const double* __restrict__ rho,
                                                     double* __restrict__ rho_old, int* __restrict__ kit,
                                                     int* __restrict__ done, int* __restrict__ iters,
-                                                    double* __restrict__ errs, int* __restrict__ active) {
+                                                    double* __restrict__ errs, const double* __restrict__ num,
+                                                    const double* __restrict__ den, double* __restrict__ alpha,
+                                                    int* __restrict__ active) {
   __shared__ double lds[BS / 64];
   double cnt = 0.0;
   for (int c = threadIdx.x; c < ncol; c += BS) {
+    const double dn = den[c];
+    alpha[c] = (done[c] || dn == 0.0) ? 0.0 : num[c] / dn;
     if (done[c]) continue;
     const int k = kit[c] + 1;
     kit[c] = k;
@@ -1028,7 +1107,8 @@ class MultiT : public MultiEngine {
     ncol_ = G_ * NB;
     for (int i = 0; i < NSC; ++i) sc_[i] = ar_.alloc<double>(ncol_);
     for (int i = 0; i < NIC; ++i) ic_[i] = ar_.alloc<int>(ncol_ + 1);
-    for (int i = 0; i < 6; ++i) kv_[i] = ar_.alloc<double>((size_t)n0_ * NB);
+    for (int i = 0; i < 6; ++i)  // z (3) is the fine level's own buffer in the FP32 form
+      if (i != 3 || std::is_same<V, double>::value) kv_[i] = ar_.alloc<double>((size_t)n0_ * NB);
     HIPCHECK(hipHostMalloc((void**)&hstat_, sizeof(int) * 4, hipHostMallocDefault));
     HIPCHECK(hipStreamSynchronize(s_));
     return 0;
@@ -1094,7 +1174,7 @@ class MultiT : public MultiEngine {
     mdot(kb, kb, sc_[C_BN2]);
     mdot(r, r, sc_[C_RR]);
     mstart_kernel<<<1, BS, 0, s_>>>(ncol_, eps, sc_[C_BN2], sc_[C_RR], sc_[C_BN], ic_[I_KIT], ic_[I_DONE],
-                                    ic_[I_ITERS], sc_[C_ERR], ic_[I_ACTIVE]);
+                                    ic_[I_ITERS], sc_[C_ERR], sc_[C_ALPHA], ic_[I_ACTIVE]);
     HIPCHECK(hipGetLastError());
     int active = read_active();
     int nl = 0, done_it = 0;
@@ -1113,6 +1193,8 @@ class MultiT : public MultiEngine {
         done_it += ch;
         if (read_active() == 0) break;
       }
+      mx_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, kx, kv_[4], sc_[C_ALPHA]);
+      HIPCHECK(hipGetLastError());
     }
     from_il(nrhs, kx, x, ldx);
     std::vector<int> it(ncol_);
@@ -1159,7 +1241,7 @@ class MultiT : public MultiEngine {
   }
 
  private:
-  enum { C_BN2, C_BN, C_RR, C_RHO, C_RHO_OLD, C_SIGMA, C_GAMMA, C_DELTA, C_PR, C_ERR, NSC };
+  enum { C_BN2, C_BN, C_RR, C_RHO, C_RHO_OLD, C_SIGMA, C_GAMMA, C_DELTA, C_PR, C_ERR, C_ALPHA, NSC };
   enum { I_KIT, I_DONE, I_ITERS, I_ACTIVE, NIC };
   int device_;
   hipStream_t s_ = nullptr;
@@ -1280,6 +1362,11 @@ class MultiT : public MultiEngine {
       bdia_launch<T, false>(m, x, e, dx, rpl, nb, xc);
       return;
     }
+    if (m.longrow) {
+      bspmm_long_kernel<T, E><<<m.nr, BS, 0, s_>>>(m.irp, m.ja, m.val, x, e);
+      HIPCHECK(hipGetLastError());
+      return;
+    }
     switch (rpl) {
       case 4:
         bspmm_kernel<T, 4, E><<<nb, BS, 0, s_>>>(m.nr, m.irp, m.ja, m.val, x, e, xc);
@@ -1310,6 +1397,7 @@ class MultiT : public MultiEngine {
       m.xmap = xm;
       return;
     }
+    m.longrow = m.fmt == FMT_CSR && m.nr < BLONG_MAX_ROWS && m.nnz >= (int64_t)BLONG_MIN_ROW * m.nr;
     if (m.nr < 4096 || !autotune_enabled()) return;
     // the temporaries are released also when a timing launch throws
     DevArena tmp;
@@ -1559,8 +1647,9 @@ class MultiT : public MultiEngine {
     mfin_kernel<NB><<<ncol_, BS, 0, s_>>>(bstart_, partial_, out);
     HIPCHECK(hipGetLastError());
   }
-  void mdot(const double* x, const double* y, double* out) {
-    mdot_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, x, y, partial_);
+  template <typename YT>
+  void mdot(const double* x, const YT* y, double* out) {
+    mdot_kernel<NB, YT><<<nrb_, BS, 0, s_>>>(bt_, x, y, partial_);
     mfin(out);
   }
   int read_active() {
@@ -1577,33 +1666,42 @@ class MultiT : public MultiEngine {
   // One iteration of every column (no host synchronisation).
   void iteration(int method, double eps, int itmax) {
     double* r = kv_[2];
-    double* z = kv_[3];
     double* p = kv_[4];
     double* q = kv_[5];
     double* x = kv_[1];
-    apply_il(r, z, true);  // r's FP32 copy was written by the previous residual update
-    if (method == 0) {  // CG
-      mdot(r, z, sc_[C_RHO]);
-      mp_cg_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, z, p, sc_[C_RHO], sc_[C_RHO_OLD], ic_[I_KIT], ic_[I_DONE]);
-      mv64_set(p, q);
-      mdot(p, q, sc_[C_SIGMA]);
-      mxr_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, x, r, p, q, sc_[C_RHO], sc_[C_SIGMA], ic_[I_DONE], partial_, r32());
-      mfin(sc_[C_RR]);
-      mcheck_kernel<<<1, BS, 0, s_>>>(ncol_, eps, itmax, sc_[C_RR], sc_[C_BN], sc_[C_RHO], sc_[C_SIGMA], sc_[C_RHO],
-                                      sc_[C_RHO_OLD], ic_[I_KIT], ic_[I_DONE], ic_[I_ITERS], sc_[C_ERR],
-                                      ic_[I_ACTIVE]);
-    } else {  // FCG(1)
-      mdot(q, z, sc_[C_GAMMA]);  // q of the previous iteration (unused in the first)
-      mp_fcg_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, z, p, r, sc_[C_GAMMA], sc_[C_DELTA], ic_[I_KIT], ic_[I_DONE],
-                                             partial_);
-      mfin(sc_[C_PR]);
-      mv64_set(p, q);
-      mdot(p, q, sc_[C_DELTA]);
-      mxr_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, x, r, p, q, sc_[C_PR], sc_[C_DELTA], ic_[I_DONE], partial_, r32());
-      mfin(sc_[C_RR]);
-      mcheck_kernel<<<1, BS, 0, s_>>>(ncol_, eps, itmax, sc_[C_RR], sc_[C_BN], sc_[C_DELTA], nullptr, nullptr,
-                                      nullptr, ic_[I_KIT], ic_[I_DONE], ic_[I_ITERS], sc_[C_ERR], ic_[I_ACTIVE]);
+    // r's FP32 copy was written by the previous residual update; z stays in
+    // the value type
+    const V* z;
+    if constexpr (std::is_same<V, double>::value) {
+      apply_il(r, kv_[3], true);
+      z = kv_[3];
+    } else {
+      apply_il(r, nullptr, true);
+      z = L_[0].y2l;
     }
+    double *num, *den;
+    if (method == 0) {  // CG
+      num = sc_[C_RHO];
+      den = sc_[C_SIGMA];
+      mdot(r, z, sc_[C_RHO]);
+      mp_cg_kernel<NB, V><<<nrb_, BS, 0, s_>>>(bt_, z, p, x, sc_[C_ALPHA], sc_[C_RHO], sc_[C_RHO_OLD], ic_[I_KIT],
+                                               ic_[I_DONE]);
+    } else {  // FCG(1)
+      num = sc_[C_PR];
+      den = sc_[C_DELTA];
+      mdot(q, z, sc_[C_GAMMA]);  // q of the previous iteration (unused in the first)
+      mp_fcg_kernel<NB, V><<<nrb_, BS, 0, s_>>>(bt_, z, p, x, sc_[C_ALPHA], r, sc_[C_GAMMA], sc_[C_DELTA],
+                                                ic_[I_KIT], ic_[I_DONE], partial_);
+      mfin(sc_[C_PR]);
+    }
+    mv64_set(p, q);
+    mdot(p, q, den);
+    mr_kernel<NB><<<nrb_, BS, 0, s_>>>(bt_, r, q, num, den, ic_[I_DONE], partial_, r32());
+    mfin(sc_[C_RR]);
+    mcheck_kernel<<<1, BS, 0, s_>>>(ncol_, eps, itmax, sc_[C_RR], sc_[C_BN], method == 0 ? num : den,
+                                    method == 0 ? den : nullptr, method == 0 ? num : nullptr, sc_[C_RHO_OLD],
+                                    ic_[I_KIT], ic_[I_DONE], ic_[I_ITERS], sc_[C_ERR], num, den, sc_[C_ALPHA],
+                                    ic_[I_ACTIVE]);
     HIPCHECK(hipGetLastError());
   }
 
