@@ -500,7 +500,10 @@ static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
   DevArena tmp;
   Work* w = tmp.alloc<Work>(1);
   HIPCHECK(hipMemsetAsync(w, 0, sizeof(Work), s));
-  dia_class_keys<V><<<nblk(m.nr), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep, &w->many);
+  const int few = 4 * BS, stride = std::max(1, m.nr / few);
+  dia_class_keys<V><<<nblk((m.nr + stride - 1) / stride), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep,
+                                                                       &w->many, stride);
+  dia_class_keys<V><<<nblk(m.nr), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep, &w->many, 1);
   HIPCHECK(hipGetLastError());
   int n = 0;
   HIPCHECK(hipMemcpyAsync(&n, &w->many, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -684,7 +684,9 @@ __global__ __launch_bounds__(BS) void diac_kernel(int nr, int nc, int nd, DiaOff
 
 // Row classes of a DIA operator.  Keys (hashes of a row's bits, never 0) are
 // put into an open table of DIACLS_SLOTS slots; more than 256 of them end the
-// search (many).  The numbers are then given by slot, and every row is compared
+// search (many): first over every stride-th row, so that an operator of
+// variable coefficients is left after a few thousand rows (all rows at once
+// raced for the table's slots, 2.5 ms for 72^3).  The numbers are then given by slot, and every row is compared
 // with the one that stands for its class, so that two rows of one hash are
 // found out (many).
 constexpr int DIACLS_SLOTS = 2048;
@@ -705,17 +707,18 @@ __device__ __forceinline__ uint64_t dia_row_key(int nr, int w, const S* __restri
 template <typename S>
 __global__ __launch_bounds__(BS) void dia_class_keys(int nr, int w, const S* __restrict__ val,
                                                      const S* __restrict__ d, unsigned long long* keys, int* rep,
-                                                     int* many) {
-  const int i = blockIdx.x * BS + threadIdx.x;
+                                                     int* many, int stride) {
+  const int64_t i = (int64_t)(blockIdx.x * BS + threadIdx.x) * stride;
   if (i >= nr || __hip_atomic_load(many, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > 256) return;
-  const unsigned long long key = dia_row_key(nr, w, val, d, i);
+  const unsigned long long key = dia_row_key(nr, w, val, d, (int)i);
   int s = (int)(key >> 20) & (DIACLS_SLOTS - 1);
   for (int probe = 0; probe < DIACLS_SLOTS; ++probe, s = (s + 1) & (DIACLS_SLOTS - 1)) {
+    if (keys[s] == key) return;  // (cached: a slot never changes once it is set)
     unsigned long long q = __hip_atomic_load(keys + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (q == 0) {
       q = atomicCAS(keys + s, 0ull, key);
       if (q == 0) {  // this row stands for the class
-        rep[s] = i;
+        rep[s] = (int)i;
         atomicAdd(many, 1);
         return;
       }
