@@ -305,10 +305,10 @@ __global__ __launch_bounds__(BS) void bdia_kernel(int nr, int nc, int nd, DiaOff
   }
 }
 // The same with the dots u.(what the epilogue stores), one per column (a pass
-// over two vectors fewer: 100 us for FP64 96^3 x 32, 64 with an FP32 one).  A
-// workgroup takes BDOT_T row blocks in turn, so that there is a partial sum
-// per 128 rows; partial[block*32 + column], added by mfin_kernel.
-constexpr int BDOT_T = 4;
+// over two vectors fewer: 100 us for FP64 96^3 x 32, 64 with an FP32 one);
+// partial[block*32 + column], added by mpart_kernel and mfin_kernel.  (Four
+// row blocks per workgroup in turn, for fewer partial sums: 238 us for the
+// FP64 product and its dots.)
 template <typename V, int RPL, int ND, class E>
 __global__ __launch_bounds__(BS) void bdia_dot_kernel(int nr, int nc, int nd, DiaOff off,
                                                       const V* __restrict__ val, const V* __restrict__ x, E e,
@@ -320,9 +320,8 @@ __global__ __launch_bounds__(BS) void bdia_dot_kernel(int nr, int nc, int nd, Di
   double dot[RPL];
 #pragma unroll
   for (int r = 0; r < RPL; ++r) dot[r] = 0.0;
-  for (int t = 0; t < BDOT_T; ++t) {
-    const int row = (lb * BDOT_T + t) * RPB + g;
-    if (row >= nr) break;
+  const int row = lb * RPB + g;
+  if (row < nr) {
     V acc[RPL];
     bdia_row<V, RPL, ND>(row, lane, nr, nc, nd, off, val, x, acc);
     const int64_t base = (int64_t)row * MB + lane * RPL;
@@ -332,7 +331,7 @@ __global__ __launch_bounds__(BS) void bdia_dot_kernel(int nr, int nc, int nd, Di
     const bv_t<V, RPL> y = e.template put<RPL>(row, base, a);
     const bv_t<double, RPL> w = bvld<double, RPL>(u, base);
 #pragma unroll
-    for (int r = 0; r < RPL; ++r) dot[r] += w[r] * (double)y[r];
+    for (int r = 0; r < RPL; ++r) dot[r] = w[r] * (double)y[r];
   }
   __shared__ double sh[RPB][MB];
 #pragma unroll
@@ -500,6 +499,22 @@ __global__ __launch_bounds__(BS) void mdot_kernel(const int4* __restrict__ bt, c
     acc += x[i] * (double)y[i];
   }
   col_partial<NB>(acc, partial);
+}
+
+// Many partial sums (one per 32 rows: 27648 for 96^3) into MPART of them:
+// block b adds rows [b per, (b + 1) per) of the nb x 32 array, in order within
+// each of its 8 row lanes (7 MB in 5 us; mfin_kernel's one block per column
+// reads them uncoalesced).
+constexpr int MPART = 256;
+__global__ __launch_bounds__(BS) void mpart_kernel(int nb, const double* __restrict__ partial,
+                                                   double* __restrict__ out) {
+  constexpr int RPS = BS / MB;
+  const int per = (nb + MPART - 1) / MPART, j = threadIdx.x % MB;
+  const int b1 = min(nb, ((int)blockIdx.x + 1) * per);
+  double acc = 0.0;
+#pragma unroll 8
+  for (int b = blockIdx.x * per + (int)threadIdx.x / MB; b < b1; b += RPS) acc += partial[(int64_t)b * MB + j];
+  col_partial<MB>(acc, out);
 }
 
 // One block per column: sum of the column's partials in block order.
@@ -1156,6 +1171,7 @@ class MultiT : public MultiEngine {
       for (const int nb : {bdot_blocks(akry_), bdot_blocks(L_[0].nd), bdot_blocks(L_[0].nd2)})
         npart = std::max(npart, nb);
     partial_ = ar_.alloc<double>((size_t)npart * NB);
+    if (npart > 4 * MPART) part2_ = ar_.alloc<double>((size_t)MPART * NB);
     ncol_ = G_ * NB;
     for (int i = 0; i < NSC; ++i) sc_[i] = ar_.alloc<double>(ncol_);
     for (int i = 0; i < NIC; ++i) ic_[i] = ar_.alloc<int>(ncol_ + 1);
@@ -1306,6 +1322,7 @@ class MultiT : public MultiEngine {
   int4* bt_ = nullptr;
   int* bstart_ = nullptr;
   double* partial_ = nullptr;
+  double* part2_ = nullptr;  // see mpart_kernel
   double* sc_[NSC] = {};
   int* ic_[NIC] = {};
   double* kv_[6] = {};
@@ -1382,7 +1399,7 @@ class MultiT : public MultiEngine {
   void bdia_launch_r(const DMat<T>& m, const T* x, E e, const double* u) {
     const int rpb = BS / (MB / RPL);
     if (u) {
-      const int nb = bdot_blocks(m), xc = bxchunk(m, rpb * BDOT_T, nb);
+      const int nb = bdot_blocks(m), xc = bxchunk(m, rpb, nb);
       if constexpr (HasPut<E>::value) {
         if (m.w == 7)
           bdia_dot_kernel<T, RPL, 7, E><<<nb, BS, 0, s_>>>(m.nr, m.nc, m.w, m.off, m.val, x, e, u, partial_, xc);
@@ -1406,7 +1423,7 @@ class MultiT : public MultiEngine {
   // workgroups, and sums per column, of a product with dots
   template <typename T>
   static int bdot_blocks(const DMat<T>& m) {
-    const int rows = BS / (MB / m.rpl) * BDOT_T;
+    const int rows = BS / (MB / m.rpl);
     return (m.nr + rows - 1) / rows;
   }
 
@@ -1744,7 +1761,13 @@ class MultiT : public MultiEngine {
   // the columns' sums over their system's reduction blocks, or over nb blocks
   // of the one system
   void mfin(double* out, int nb = 0) {
-    mfin_kernel<NB><<<ncol_, BS, 0, s_>>>(bstart_, nb, partial_, out);
+    const double* part = partial_;
+    if (nb > 4 * MPART) {
+      mpart_kernel<<<MPART, BS, 0, s_>>>(nb, partial_, part2_);
+      part = part2_;
+      nb = MPART;
+    }
+    mfin_kernel<NB><<<ncol_, BS, 0, s_>>>(bstart_, nb, part, out);
     HIPCHECK(hipGetLastError());
   }
   template <typename YT>
