@@ -57,6 +57,11 @@ struct DMat {
   // is column col0 + k + (dja_0 + ... + dja_k) (padding: steps of 0)
   int* col0 = nullptr;
   uint16_t* dja = nullptr;
+  // SELL, SELD of few distinct values (see sellp_kernel): column or step in
+  // the low pcb bits, number of the value in ptab (pnt of them) above
+  uint32_t* pk = nullptr;
+  V* ptab = nullptr;
+  int pnt = 0, pcb = 0;
   int* ja = nullptr;
   V* val = nullptr;
   // DIA with at most 256 distinct rows: class of each row, the classes'
@@ -579,6 +584,61 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
   red_finish<K>(red, nb, s);
 }
 
+// SELL, SELD operators whose values are few: packed words beside the arrays
+// (see sellp_kernel).  From 32768 rows, as the DIA classes: below, an operator
+// lies in the caches and its product takes the time of its gathers.  Tables of
+// more than 1024 values where 512 rows and more share one: loading the table
+// is then hidden by the other workgroups of the launch.
+constexpr int DICT_MIN_ROWS = 32768;
+template <typename V>
+static void value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
+  m.pk = nullptr;
+  if ((m.fmt != FMT_SELL && m.fmt != FMT_SELD) || m.nr < DICT_MIN_ROWS || m.stored < 1) return;
+  int cb = 16;
+  if (m.fmt == FMT_SELL)
+    for (cb = 1; cb < 31 && ((int64_t)1 << cb) < m.nc; ++cb) {}
+  struct Work {
+    unsigned long long keys[DICT_SLOTS];
+    int num[DICT_SLOTS], many;
+  };
+  DevArena tmp;
+  Work* w = tmp.alloc<Work>(1);
+  HIPCHECK(hipMemsetAsync(w, 0, sizeof(Work), s));
+  auto blocks = [](int64_t n) { return (int)((n + BS - 1) / BS); };
+  const int stride = (int)std::max<int64_t>(1, m.stored / (64 * BS));
+  dict_keys<V><<<blocks((m.stored + stride - 1) / stride), BS, 0, s>>>(m.stored, m.val, w->keys, &w->many, stride);
+  dict_keys<V><<<blocks(m.stored), BS, 0, s>>>(m.stored, m.val, w->keys, &w->many, 1);
+  HIPCHECK(hipGetLastError());
+  int n = 0;
+  HIPCHECK(hipMemcpyAsync(&n, &w->many, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIPCHECK(hipStreamSynchronize(s));
+  if (n < 1 || n > std::min(DICT_MAX, std::max(1024, m.nr / 512)) || (int64_t)n > ((int64_t)1 << (32 - cb))) return;
+  m.ptab = ar.alloc<V>(n);
+  m.pk = ar.alloc<uint32_t>((size_t)m.stored);
+  m.pnt = n;
+  m.pcb = cb;
+  dict_number<V><<<1, BS, 0, s>>>(w->keys, w->num, m.ptab);
+  dict_pack<V><<<blocks(m.stored), BS, 0, s>>>(m.stored, m.val, m.ja, m.fmt == FMT_SELD ? m.dja : nullptr, w->keys,
+                                               w->num, cb, m.pk);
+  HIPCHECK(hipGetLastError());
+  HIPCHECK(hipStreamSynchronize(s));  // before tmp is released
+  if (std::getenv("MLD_VERBOSE"))
+    std::fprintf(stderr, "[mld] %d x %d operator (%s): %d distinct values\n", m.nr, m.nc,
+                 m.fmt == FMT_SELL ? "SELL" : "SELD", n);
+}
+template <typename C, typename V, class G, class E>
+static void sellp_launch(const DMat<V>& m, G g, E e, hipStream_t s) {
+  const int nb = (m.nr + BS - 1) / BS, xc = xcd_chunk(m.xmap, nb, BS);
+  const size_t lds = (size_t)m.pnt * sizeof(V);
+  if (m.fmt == FMT_SELD)
+    sellp_kernel<C, true><<<nb, BS, lds, s>>>(m.nr, m.nc, m.sptr, m.perm, m.col0, m.pk, m.ptab, m.pnt, m.pcb, g, e,
+                                              xc);
+  else
+    sellp_kernel<C, false><<<nb, BS, lds, s>>>(m.nr, m.nc, m.sptr, m.perm, nullptr, m.pk, m.ptab, m.pnt, m.pcb, g,
+                                               e, xc);
+  HIPCHECK(hipGetLastError());
+}
+
 template <int K = 0, typename CT = void, typename V, class G, class E>
 static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red{}) {
   using C = typename std::conditional<std::is_void<CT>::value, V, CT>::type;
@@ -592,6 +652,12 @@ static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red
     }
     dia_launch<K, C>(m, g, e, s, red);
     return;
+  }
+  if constexpr (K == 0) {
+    if (m.pk) {
+      sellp_launch<C>(m, g, e, s);
+      return;
+    }
   }
   const int nb = spmv_blocks(m);
   red_fuse(red, nb);

@@ -50,11 +50,14 @@ class DevPrecT : public DevPrec {
       double t0 = wall_seconds();
       D.a = upload_tuned<V>(H.a, ar_, s_, p.dev_format);
       dia_classes<V>(D.a, nullptr, ar_, s_);
+      value_dictionary<V>(D.a, ar_, s_);
       phase_log("upload A", l + 1, wall_seconds() - t0);
       if (l > 0) {
         t0 = wall_seconds();
         D.p = upload_tuned<V>(H.p, ar_, s_, p.dev_format);
         D.r = upload_tuned<V>(H.r, ar_, s_, p.dev_format);
+        value_dictionary<V>(D.p, ar_, s_);
+        value_dictionary<V>(D.r, ar_, s_);
         phase_log("upload P, R", l + 1, wall_seconds() - t0);
       }
       t0 = wall_seconds();
@@ -701,6 +704,8 @@ class DevPrecT : public DevPrec {
       HIPCHECK(hipGetLastError());
       dia_classes<V>(S.nd, S.dv, ar_, s_);
       dia_classes<V>(S.ndd, S.dv, ar_, s_);
+      value_dictionary<V>(S.nd, ar_, s_);
+      value_dictionary<V>(S.ndd, ar_, s_);
     }
     if (H.solver == ILU_N || H.solver == GS || H.solver == BWGS) {
       S.l = upload_mat<V>(H.l, ar_, s_, 1, 1);  // CSR (rows summed in stored order)
