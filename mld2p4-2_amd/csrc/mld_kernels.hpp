@@ -1475,6 +1475,11 @@ __global__ __launch_bounds__(BS) void trsv_sf_kernel(int nchunks, const int* __r
 // read and write 64 consecutive values instead of one value in each of 64
 // grid lines; grid_to_steps_kernel / grid_from_steps_kernel convert the
 // input and the output.
+// Bound by the chain through the tiles, nx + 14 steps in each and one face to
+// cross per tile of a row and a column: a step is then two cross-lane reads and
+// three products, and memory latency must not be on it.  So operands and faces
+// are loaded GRID_P steps ahead.
+constexpr int GRID_P = 8;
 template <typename V, int SC, bool BACK>
 __global__ __launch_bounds__(64) void trsv_grid_kernel(int nx, int ny, int nz, int64_t sz, const V* __restrict__ g,
                                                        const V* __restrict__ d, const V* __restrict__ b, V* t,
@@ -1508,32 +1513,103 @@ __global__ __launch_bounds__(64) void trsv_grid_kernel(int nx, int ny, int nz, i
                              : base - ns * 64 + (int64_t)(7 + kk) * 64 + 7 + 8 * kk;
     const int64_t fk0 = BACK ? base + (int64_t)ntj * ns * 64 + (int64_t)jj * 64 + jj
                              : base - (int64_t)ntj * ns * 64 + (int64_t)(jj + 7) * 64 + jj + 56;
-    V prev = (V)0;
-    for (int st = 0; st < nx + 14; ++st) {
-      const V vj = __shfl(prev, ljn), vk = __shfl(prev, lkn);
-      const int mi = st - mj - mk;
-      if (valid && mi >= 0 && mi < nx) {
-        const int i = BACK ? nx - 1 - mi : mi;
-        const int64_t q = base + (int64_t)(i + jj + kk) * 64 + lane;  // this point's position
-        const bool hasi = BACK ? i + 1 < nx : i > 0;
-        const V g0 = g[q], g1 = g[sz + q], g2 = g[2 * sz + q];
-        const V bi = (SC == 1) ? d[q] * b[q] : b[q];
-        const V tj = facej ? sf_wait(t + fj0 + (int64_t)i * 64, abort, spin_max) : vj;
-        const V tk = facek ? sf_wait(t + fk0 + (int64_t)i * 64, abort, spin_max) : vk;
-        V acc = (V)0;
-        if (!BACK) {
-          if (hask) acc = acc + g0 * tk;
-          if (hasj) acc = acc + g1 * tj;
-          if (hasi) acc = acc + g2 * prev;
-        } else {
-          if (hasi) acc = acc + g0 * prev;
-          if (hasj) acc = acc + g1 * tj;
-          if (hask) acc = acc + g2 * tk;
-        }
-        const V ti = (SC == 2) ? (bi - acc) / d[q] : bi - acc;
-        __hip_atomic_store(t + q, ti, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        prev = ti;
+    // GRID_P steps' operands and face values, loaded one batch ahead
+    struct Batch {
+      V g0[GRID_P], g1[GRID_P], g2[GRID_P], b[GRID_P], d[GRID_P], tj[GRID_P], tk[GRID_P];
+    };
+    const V* const own = t + base;  // what a lane without such a neighbour reads
+    auto face = [&](bool need, int64_t f0, int st) {
+      const int mi = min(max(st - mj - mk, 0), nx - 1);
+      const V* p = need ? t + f0 + (int64_t)(BACK ? nx - 1 - mi : mi) * 64 : own;
+      return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto load = [&](Batch& B, int s0) {
+#pragma unroll
+      for (int u = 0; u < GRID_P; ++u) {
+        const int st = min(s0 + u, (int)ns - 1);
+        const int64_t q = base + (BACK ? ns - 1 - st : (int64_t)st) * 64 + lane;
+        B.g0[u] = g[q];
+        B.g1[u] = g[sz + q];
+        B.g2[u] = g[2 * sz + q];
+        B.b[u] = b[q];
+        B.d[u] = SC == 0 ? (V)1 : d[q];
       }
+#pragma unroll
+      for (int u = 0; u < GRID_P; ++u) {
+        B.tj[u] = face(facej, fj0, s0 + u);
+        B.tk[u] = face(facek, fk0, s0 + u);
+      }
+    };
+    V prev = (V)0;
+    auto steps = [&](Batch& B, int s0) {
+#pragma unroll
+      for (int u = 0; u < GRID_P; ++u) {
+        const int st = s0 + u;
+        if (st >= (int)ns) break;
+        const V vj = __shfl(prev, ljn), vk = __shfl(prev, lkn);
+        const int mi = st - mj - mk;
+        const bool act = valid && mi >= 0 && mi < nx;
+        // values that were not there yet when the batch was loaded: all that
+        // it has left are loaded again
+        auto miss = [&]() {
+          return __any(act && ((facej && SfSentinel<V>::is(B.tj[u])) || (facek && SfSentinel<V>::is(B.tk[u]))));
+        };
+        if (miss()) {
+          int n = 0;
+          do {
+            const bool stop =
+                n++ >= spin_max || __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0.0;
+            if (__any(stop)) {
+              __hip_atomic_store(abort, 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+              for (int w = u; w < GRID_P; ++w) {
+                if (SfSentinel<V>::is(B.tj[w])) B.tj[w] = (V)0;
+                if (SfSentinel<V>::is(B.tk[w])) B.tk[w] = (V)0;
+              }
+              break;
+            }
+#pragma unroll
+            for (int w = u; w < GRID_P; ++w) {
+              B.tj[w] = face(facej, fj0, s0 + w);
+              B.tk[w] = face(facek, fk0, s0 + w);
+            }
+            // (vmcnt(0), here, so that the code after the block does not have
+            // to assume loads younger than the next batch's)
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+          } while (miss());
+        }
+        if (act) {
+          const int i = BACK ? nx - 1 - mi : mi;
+          const bool hasi = BACK ? i + 1 < nx : i > 0;
+          const V bi = (SC == 1) ? B.d[u] * B.b[u] : B.b[u];
+          const V tj = facej ? B.tj[u] : vj;
+          const V tk = facek ? B.tk[u] : vk;
+          V acc = (V)0;
+          if (!BACK) {
+            if (hask) acc = acc + B.g0[u] * tk;
+            if (hasj) acc = acc + B.g1[u] * tj;
+            if (hasi) acc = acc + B.g2[u] * prev;
+          } else {
+            if (hasi) acc = acc + B.g0[u] * prev;
+            if (hasj) acc = acc + B.g1[u] * tj;
+            if (hask) acc = acc + B.g2[u] * tk;
+          }
+          const V ti = (SC == 2) ? (bi - acc) / B.d[u] : bi - acc;
+          __hip_atomic_store(t + base + (int64_t)(i + jj + kk) * 64 + lane, ti, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+          prev = ti;
+        }
+      }
+    };
+    Batch B0, B1;
+    load(B0, 0);
+    // (loads past the last step repeat it: under a condition, the code after
+    // them would wait as if they had not been issued)
+    for (int s0 = 0; s0 < (int)ns; s0 += 2 * GRID_P) {
+      load(B1, s0 + GRID_P);
+      steps(B0, s0);
+      load(B0, s0 + 2 * GRID_P);
+      steps(B1, s0 + GRID_P);
     }
   }
 }
