@@ -86,13 +86,13 @@ def level_table(p):
                  solver=i["solver"], sweeps_pre=i["sweeps_pre"], sweeps_post=i["sweeps_post"])
         fa = p.op_format(l, "A")
         d["csr_a"] = fa["fmt"] == "CSR"
-        d["fmt_a"] = fa["fmt"]
+        d["fmt_a"] = p.op_bytes_form(l, "A")
         if l > 0:
-            d["fmt_p"] = p.op_format(l, "P")["fmt"]
-            d["fmt_r"] = p.op_format(l, "R")["fmt"]
+            d["fmt_p"] = p.op_bytes_form(l, "P")
+            d["fmt_r"] = p.op_bytes_form(l, "R")
         if i["nnz_nd"] > 0:
             d["csr_nd"] = p.op_format(l, "ND")["fmt"] == "CSR"
-            d["fmt_nd"] = p.op_format(l, "ND")["fmt"]
+            d["fmt_nd"] = p.op_bytes_form(l, "ND")
         if i["solver"] == 7:
             d["nnz_lu"] = p.level_csr(l, "L").nnz + p.level_csr(l, "U").nnz
         levels.append(d)

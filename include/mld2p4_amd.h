@@ -292,6 +292,11 @@ int mldhip_time_step(mldhip_prec* p, int lev, int kind, int reps, double* avg_ms
  * fmt 0 = CSR with `lanes` lanes per row, 1 = ELL of width `width`, 2 = SELL,
  * 3 = DIA with `width` diagonals, 4 = SELL with 16-bit column steps. */
 int mldhip_get_op_format(mldhip_prec* p, int lev, int what, int* fmt, int* lanes, int* width);
+/* What products of that operator read instead of its values (ND: of ND D):
+ * kind 0 nothing else, 1 a byte per row naming its class (DIA), 2 a 32-bit
+ * word per entry with the number of its value (SELL, SELD).  No reference
+ * counterpart (byte counts). */
+int mldhip_get_op_packed(mldhip_prec* p, int lev, int what, int* kind);
 
 #ifdef __cplusplus
 }

@@ -90,6 +90,7 @@ def lib():
             "mldhip_level_smooth": [vp, C.c_int, C.c_int, vp, C.c_int, vp, C.c_int, C.c_char],
             "mldhip_time_step": [vp, C.c_int, C.c_int, C.c_int, dp],
             "mldhip_get_op_format": [vp, C.c_int, C.c_int, ip, ip, ip],
+            "mldhip_get_op_packed": [vp, C.c_int, C.c_int, ip],
             "mldhip_krylov_adjoint": [vp, cp, vp, vp, C.c_double, C.c_int, C.c_int, ip, dp],
             "mldhip_fv7_grad_theta": [C.c_int, vp, vp, vp, vp, vp, vp],
             "mldhip_apply_block": [vp, C.c_int, vp, C.c_int64, vp, C.c_int64],
@@ -455,6 +456,13 @@ class MldPrec:
         self._check(lib().mldhip_get_op_format(self.h, lev, LEVEL_OPS[what], C.byref(f), C.byref(l), C.byref(w)),
                     "get_op_format")
         return {"fmt": ("CSR", "ELL", "SELL", "DIA", "SELD")[f.value], "lanes": l.value, "width": w.value}
+
+    def op_bytes_form(self, lev, what):
+        """The layout's name for byte counts: DIA, SELL or SELD with "+rows" or "+values" where products read row
+        classes or packed words."""
+        k = C.c_int()
+        self._check(lib().mldhip_get_op_packed(self.h, lev, LEVEL_OPS[what], C.byref(k)), "get_op_packed")
+        return self.op_format(lev, what)["fmt"] + ("", "+rows", "+values")[k.value]
 
     def level_smooth(self, lev, x, y, beta=0, sweeps=1, trans="N", which=0):
         self.use_torch_stream()

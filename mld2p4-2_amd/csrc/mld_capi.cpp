@@ -502,6 +502,13 @@ int mldhip_get_op_format(mldhip_prec* p, int lev, int what, int* fmt, int* lanes
   return p->dev->op_format(lev, what, fmt, lanes, width);
 }
 
+int mldhip_get_op_packed(mldhip_prec* p, int lev, int what, int* kind) {
+  int rc = need_dev(p);
+  if (rc) return rc;
+  if (!kind) return E_BAD_ARG;
+  return p->dev->op_packed(lev, what, kind);
+}
+
 // ---- batched engines --------------------------------------------------------
 static int ensure_block(mldhip_prec* p) {
   int rc = need_dev(p);

@@ -510,6 +510,16 @@ class DevPrecT : public DevPrec {
     return 0;
   }
 
+  int op_packed(int lev, int what, int* kind) override {
+    if (lev < 0 || lev >= (int)L_.size()) return E_BAD_LEVEL;
+    DLevel<V>& D = L_[lev];
+    if (what < 0 || what > 3) return E_BAD_ARG;
+    // ND: the form of ND D, which the sweeps from zero multiply by
+    const DMat<V>& m = what == 0 ? D.a : what == 1 ? D.p : what == 2 ? D.r : D.sm.ndd.val ? D.sm.ndd : D.sm.nd;
+    *kind = m.cls ? 1 : m.pk ? 2 : 0;
+    return 0;
+  }
+
   int time_step(int lev, int kind, int reps, double* avg_ms) override {
     HIPCHECK(hipSetDevice(device_));
     if (lev < 0 || lev >= (int)L_.size() || reps <= 0) return E_BAD_LEVEL;

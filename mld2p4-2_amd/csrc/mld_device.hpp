@@ -40,6 +40,7 @@ class DevPrec {
   virtual int time_step(int lev, int kind, int reps, double* avg_ms) = 0;
   // Storage chosen for a level operator: fmt (0 CSR, 1 ELL), lanes, width.
   virtual int op_format(int lev, int what, int* fmt, int* lanes, int* width) = 0;
+  virtual int op_packed(int lev, int what, int* kind) = 0;
 };
 
 DevPrec* make_dev_prec(int value_kind, int device, hipStream_t stream);

@@ -16,6 +16,10 @@ def mat_bytes(nr, nnz, sv, fmt):
     """Compulsory bytes of one pass over a stored operator: values and column
     indices (CSR also row pointers; DIA stores no indices; SELD stores 16-bit
     column steps and one 32-bit first column per row)."""
+    if fmt == "DIA+rows":  # one byte per row naming its class
+        return nr
+    if fmt in ("SELL+values", "SELD+values"):  # one word per entry; SELD: and the first column
+        return nnz * 4 + (nr * 4 if fmt == "SELD+values" else 0)
     if fmt == "DIA":
         return nnz * sv
     if fmt == "SELD":
@@ -45,8 +49,9 @@ def smoother_bytes(n, solver, sweeps, nnz_nd, nnz_lu, sv, sx, beta, nd_csr=False
         if sweeps <= 1 or nnz_nd == 0:
             return 2 * n * sx * nb + n * sv + yread  # y = d*x
         m = mat_bytes(n, nnz_nd, sv, nd_fmt or ("CSR" if nd_csr else "ELL"))
-        first = m + n * (2 * sx * nb + sv)  # D^-1(x - ND D^-1 x)
-        more = (sweeps - 2) * (m + n * (3 * sx * nb + sv))
+        sd = 0 if nd_fmt == "DIA+rows" else sv  # (d_i is in the row's class)
+        first = m + n * (2 * sx * nb + sd)  # D^-1(x - ND D^-1 x)
+        more = (sweeps - 2) * (m + n * (3 * sx * nb + sd))
         return first + more + yread
     if solver == ILU_N:
         return nnz_lu * (sv + 4) + 2 * (n + 1) * 4 + n * sv + 4 * n * sx + yread
