@@ -466,9 +466,14 @@ struct has_pair : std::false_type {};
 template <class E>
 struct has_pair<E, std::void_t<decltype(std::declval<const E&>().aligned2())>> : std::true_type {};
 
-// The end of a reduction over nb blocks: in the kernel itself (red_fuse left
-// the ticket), or by finalize_kernel.
+// A reduction of K sums over nb blocks: every one writes its partial sums, so
+// they have to fit.  It ends in the kernel itself (red_fuse left the ticket),
+// or by finalize_kernel.
+template <int K>
 static inline void red_fuse(Red& red, int nb) {
+  if (K > 0 && (int64_t)K * nb > red.cap)
+    throw DevError("a reduction over " + std::to_string(nb) + " blocks with room for " + std::to_string(red.cap) +
+                   " partial sums");
   if (nb > RED_FUSE_MAX) red.ticket = nullptr;
 }
 template <int K>
@@ -550,7 +555,7 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
       constexpr int RPB = 2 * DIACLS_P * BS;
       const int nbp = (int)(((int64_t)m.nr + RPB - 1) / RPB);
       const int xc = xcd_chunk(m.xmap, nbp, RPB);
-      red_fuse(red, nbp);
+      red_fuse<K>(red, nbp);
       if (m.w == 7)
         diac_kernel<C, 7, K, D><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.cls, m.ctab, m.cdef, g.x, e, red, xc);
       else
@@ -566,7 +571,7 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
     if ((m.nr & 1) == 0 && al2(m.val, sizeof(V)) && e.aligned2()) {
       const int nbp = (int)(((int64_t)m.nr / 2 + BS - 1) / BS);
       const int xc = xcd_chunk(m.xmap, nbp, 2 * BS);
-      red_fuse(red, nbp);
+      red_fuse<K>(red, nbp);
       if (m.w == 7)
         dia_kernel<C, 7, K, 1, G, E, V, true><<<nbp, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
       else
@@ -578,7 +583,7 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
   constexpr int RPT = dia_rpt<K>();
   const int nb = (int)(((int64_t)m.nr + BS * RPT - 1) / (BS * RPT));
   const int xc = xcd_chunk(m.xmap, nb, BS * RPT);
-  red_fuse(red, nb);
+  red_fuse<K>(red, nb);
   if (m.w == 7) dia_kernel<C, 7, K, RPT><<<nb, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
   else dia_kernel<C, 0, K, RPT><<<nb, BS, 0, s>>>(m.nr, m.nc, m.w, m.off, m.val, g, e, red, xc);
   red_finish<K>(red, nb, s);
@@ -660,7 +665,7 @@ static void spmv_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red = Red
     }
   }
   const int nb = spmv_blocks(m);
-  red_fuse(red, nb);
+  red_fuse<K>(red, nb);
   if (m.fmt == FMT_ELL) {
     const int xc = xcd_chunk(m.xmap, nb, BS);
     switch (m.w) {

@@ -110,7 +110,7 @@ class DevPrecT : public DevPrec {
       nbmax = std::max(nbmax, nblk(n0_));
       for (auto& D : L_)
         if (D.kd0) nbmax = std::max(nbmax, spmv_blocks(D.a));
-      partial_ = ar_.alloc<double>(2 * (size_t)nbmax + 64);
+      reserve_partials(nbmax);
     }
     ticket_ = ar_.alloc<int>(RED_TICKETS);
     HIPCHECK(hipMemsetAsync(ticket_, 0, RED_TICKETS * sizeof(int), s_));
@@ -633,11 +633,22 @@ class DevPrecT : public DevPrec {
     else spmv_launch<K>(akry_, g, e, s_, r);
   }
   bool akry_t_set_ = false;
+  // Partial sums of the reducing launches, two of each of at most nb blocks.
+  // Operators that are uploaded later (transposes, whose rows need not be as
+  // long as A's, so neither as many lanes) ask for theirs; launches under way
+  // keep the array that they were given.
   double* partial_ = nullptr;
+  int64_t partial_cap_ = 0;
+  void reserve_partials(int nb) {
+    const int64_t want = 2 * (int64_t)nb + 64;
+    if (want <= partial_cap_) return;
+    partial_ = ar_.alloc<double>((size_t)want);
+    partial_cap_ = want;
+  }
   // reduction into slot; publish: its end also sends every slot to the host,
   // which waits for them in read_scal
   Red red(int slot, bool publish = false) {
-    Red r{partial_, scal_ + slot, ticket_, scal_, nullptr, 0};
+    Red r{partial_, scal_ + slot, ticket_, scal_, nullptr, 0, partial_cap_};
     if (publish) {
       r.host = hscal_;
       r.seq = ++seq_;
@@ -648,7 +659,7 @@ class DevPrecT : public DevPrec {
   // many (red_finish then adds the partial sums)
   Red red_for(int slot, int nb, bool publish = false) {
     Red r = red(slot, publish);
-    red_fuse(r, nb);
+    red_fuse<2>(r, nb);  // (of one or two sums)
     return r;
   }
   int* ticket_ = nullptr;  // see block_partials
@@ -907,6 +918,8 @@ class DevPrecT : public DevPrec {
       tsm(H.smd, D.sm);
       if (D.has_sm2) tsm(H.smd2, D.sm2);
     }
+    // the fine level's last sweep of an application with a dot
+    reserve_partials(std::max(spmv_blocks(L_[0].sm.ndt), spmv_blocks(L_[0].sm2.ndt)));
     build_tail_t();
     transposes_ = true;
   }
@@ -1723,10 +1736,11 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
       } else {
         akry_t_ = upload_mat<double>(host_transpose(hprec_->precv[0].a), ar_, s_, hprec_->dev_format);
       }
+      reserve_partials(spmv_blocks(akry_t_));
       akry_t_set_ = true;
     }
   }
-    double* r = kvec(0);
+  double* r = kvec(0);
   double* z = kvec(1);
   double* p = kvec(2);
   double* q = kvec(3);

@@ -294,6 +294,7 @@ struct Red {  // reduction buffers of a kernel with dot outputs
   const double* scal;  // with host: the scalar slots go to host[0..S_NSCAL) when the sums are
   double* host;        // done, then seq to host[S_NSCAL] (pinned memory; the host waits for it)
   unsigned long long seq;
+  int64_t cap;  // doubles in partial (checked on the host, see red_fuse)
 };
 // Scalar slots in device memory.
 enum { S_RHO0 = 0, S_RHO1 = 1, S_SIGMA = 2, S_RR = 3, S_PR = 4, S_GAMMA = 5, S_DELTA = 6, S_DPR = 7,
