@@ -494,13 +494,19 @@ template <typename V, typename XT>
 struct gather_x<GatherX<V, XT>> : std::true_type {};
 
 // Row classes of a DIA operator (see diac_kernel), d: the smoother's diagonal
-// (null: not used with it).  Left out below DIACLS_MIN_ROWS rows, where the
-// values stay in the caches.
-constexpr int DIACLS_MIN_ROWS = 32768;
+// (null: not used with it).  Only where the stored values take at least
+// DIACLS_MIN_BYTES: fewer stay in the caches, and reading them is then quicker
+// than the classes' table behind a barrier.  7-point levels, V-cycles with
+// l1-Jacobi 2/2, with stored values -> with classes: FP64 48^3 (6.2 MB) 53.9 ->
+// 55.2 us, 50^3 (7.0 MB) 61.6 -> 61.7, 52^3 (7.9 MB) 65.1 -> 63.0, 56^3 69.9 ->
+// 66.9; FP32 56^3 (4.9 MB) 55.2 -> 57.7, 60^3 (6.0 MB) 60.7 -> 62.0, 64^3 (7.3
+// MB) 65.2 -> 65.1, 72^3 (10.5 MB) 82.2 -> 81.3; at 33^3 the residual alone 2.6
+// -> 3.6 us.
+constexpr double DIACLS_MIN_BYTES = 7e6;
 template <typename V>
 static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
   m.cls = nullptr;
-  if (m.fmt != FMT_DIA || m.nr < DIACLS_MIN_ROWS || m.w < 1 || (d && m.w > 7)) return;
+  if (m.fmt != FMT_DIA || m.w < 1 || (d && m.w > 7) || (double)m.nr * m.w * sizeof(V) < DIACLS_MIN_BYTES) return;
   struct Work {  // one allocation; from tab on copied back together
     unsigned long long keys[DIACLS_SLOTS];
     int rep[DIACLS_SLOTS], num[DIACLS_SLOTS];
