@@ -9,7 +9,6 @@
 #include <algorithm>
 #include <cmath>
 #include <atomic>
-#include <future>
 #include <cstdio>
 #include <thread>
 #include <cstdlib>
@@ -798,12 +797,8 @@ class DevPrecT : public DevPrec {
     const bool ilu = (H.solver == ILU_N);
     tp::Packed<V> pl, pu;
     const double* d = H.dv.empty() ? nullptr : H.dv.data();
-    // (both factors at once; an exception of the second thread arrives by get())
-    auto second = std::async(ilu ? std::launch::async : std::launch::deferred, [&] {
-      return H.solver == GS || tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu);
-    });
-    const bool okl = H.solver == BWGS || tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl);
-    if (!second.get() || !okl) return;
+    if (H.solver != BWGS && !tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl)) return;
+    if (H.solver != GS && !tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu)) return;
     std::vector<int> pos(n), idx(n);
     auto up = [&](const tp::Packed<V>& f, typename DSmoother<V>::PackedTri& t) {
       for (int p = 0; p < n; ++p) pos[f.rows[p]] = p;

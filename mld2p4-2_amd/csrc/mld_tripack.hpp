@@ -24,145 +24,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cstdint>
-#include <cstring>
 #include <type_traits>
-#include <vector>
 
-#include "mld_host.hpp"
 #include "mld_kernels.hpp"
+#include "mld_tripack_host.hpp"
 
 namespace mld {
 namespace tp {
-
-constexpr int TP_NW = 12;                 // wavefronts
-constexpr int TP_T = 64 * TP_NW;
-constexpr int TP_KE = 16;                 // entries of a row in registers that are summed ahead of its group
-constexpr int TP_KL = 24;                 // and behind the barrier
-constexpr int TP_LDS = 160 * 1024;        // the whole LDS of a CU
-
-// Rows whose solution the LDS window holds; behind them a constant zero, which
-// padding entries point to, and a slot that nobody reads.
-template <typename V>
-constexpr int tp_w() { return (TP_LDS - 64) / (int)sizeof(V) < 32766 ? (TP_LDS - 64) / (int)sizeof(V) : 32766; }
-template <typename V>
-constexpr int tp_vpc() { return 16 / (int)sizeof(V); }  // values of a 16-byte chunk
-
-struct SliceHdr {
-  uint32_t off;   // data offset, 16-byte units
-  int32_t p;      // first position
-  int32_t g;      // group
-  uint32_t shape; // 15 bits: p mod window; 6: rows - 1; 3: chunks of 4 entries summed ahead; 8: chunks
-};
-
-template <typename V>
-struct Packed {
-  std::vector<unsigned char> bytes;  // slice data
-  std::vector<SliceHdr> hdr;         // slices of wavefront 0, of wavefront 1, ...; each list ends with two of group ngroups
-  std::vector<int> first;            // TP_NW + 1 starts in hdr
-  std::vector<int> rows;             // position -> row
-  int ngroups = 0;
-};
-
-// Data bytes of a slice: columns (slots) in chunks of 4, values in 16-byte
-// chunks (rows padded to 4 entries), both chunk-major over the rows, then the
-// diagonal.
-template <typename V>
-static inline size_t tp_slice_bytes(int m, int w) {
-  const size_t c = (w + 3) / 4, q = c * 4 / tp_vpc<V>();
-  return (c * m * 8 + 15) / 16 * 16 + q * m * 16 + (sizeof(V) * m + 15) / 16 * 16;
-}
-
-// The packed form of factor f (level sets ptr / rows), diagonal d (null: none
-// is read).  False when a dependency lies outside the window, a row is too
-// long, or the stream (at the 90 GB/s of one CU) takes longer than the waits
-// it saves: the sync-free form spends 1.3 to 1.65 us on a level set of these
-// widths and spreads the bytes over the whole GPU, so the line lies at 1.2 us
-// of stream per level set (the first coarse level of a 256^3 grid, 905 rows
-// of 15 entries per level set, stays sync-free: 3.3 ms of stream against
-// 3.7 ms).
-template <typename V>
-static bool tp_pack(const HCsr& f, const std::vector<int>& ptr, const std::vector<int>& srows, const double* d,
-                    Packed<V>& out) {
-  const int n = f.nr, nlev = (int)ptr.size() - 1;
-  constexpr int W = tp_w<V>();
-  if (n <= 0 || nlev <= 0) return false;
-  const double us = ((double)f.nnz() * (sizeof(V) + 2) * 1.2 + (double)n * (2 * sizeof(V))) / 90e3;
-  if (us > 1.2 * nlev) return false;
-  out.rows = srows;
-  std::vector<int>& rows = out.rows;
-  auto len = [&](int r) { return (int)(f.irp[r + 1] - f.irp[r]); };
-  std::vector<int> pos(n);
-  for (int l = 0; l < nlev; ++l) {
-    std::stable_sort(rows.begin() + ptr[l], rows.begin() + ptr[l + 1], [&](int a, int b) { return len(a) > len(b); });
-    for (int p = ptr[l]; p < ptr[l + 1]; ++p) pos[rows[p]] = p;
-    if (ptr[l + 1] > ptr[l] && len(rows[ptr[l]]) > 1000) return false;
-  }
-  // the window: a row reads slots of positions that no row of its level set,
-  // or of an earlier one, has taken since
-  for (int l = 0; l < nlev; ++l)
-    for (int p = ptr[l]; p < ptr[l + 1]; ++p) {
-      const int r = rows[p];
-      for (int64_t k = f.irp[r]; k < f.irp[r + 1]; ++k)
-        if (pos[f.ja[k]] >= ptr[l] || ptr[l + 1] - 1 - pos[f.ja[k]] >= W) return false;
-    }
-  out.bytes.clear();
-  std::vector<std::vector<SliceHdr>> list(TP_NW);
-  std::vector<int> gg(n);  // position -> group
-  int G = -1, turn = 0;
-  for (int l = 0; l < nlev; ++l) {
-    int ingroup = TP_NW;
-    for (int p = ptr[l]; p < ptr[l + 1];) {
-      if (ingroup == TP_NW) {
-        ++G;
-        ingroup = 0;
-      }
-      const int m = std::min(64, ptr[l + 1] - p), w = len(rows[p]);
-      const int nc = (w + 3) / 4, nq = nc * 4 / tp_vpc<V>();
-      // leading chunks of 4 entries without one from the group before
-      int ke = std::min(nc, TP_KE / 4);
-      for (int i = p; i < p + m; ++i) {
-        gg[i] = G;
-        const int64_t k0 = f.irp[rows[i]];
-        for (int k = 0; k < std::min(4 * ke, len(rows[i])); ++k)
-          if (gg[pos[f.ja[k0 + k]]] >= G - 1) ke = k / 4;
-      }
-      const size_t base = out.bytes.size();
-      if (base / 16 > 0xf0000000ull) return false;
-      out.bytes.resize(base + tp_slice_bytes<V>(m, w), 0);
-      uint16_t* col = (uint16_t*)(out.bytes.data() + base);
-      V* val = (V*)(out.bytes.data() + base + ((size_t)nc * m * 8 + 15) / 16 * 16);
-      V* dd = val + (size_t)nq * m * tp_vpc<V>();
-      for (int i = 0; i < m; ++i) {
-        const int r = rows[p + i], ln = len(r);
-        const int64_t k0 = f.irp[r];
-        // padding: -0 times the zero slot is -0, and acc + (-0) = acc
-        for (int k = 0; k < nc * 4; ++k) {
-          col[((size_t)(k / 4) * m + i) * 4 + k % 4] = (uint16_t)(k < ln ? pos[f.ja[k0 + k]] % W : W);
-          val[((size_t)(k / tp_vpc<V>()) * m + i) * tp_vpc<V>() + k % tp_vpc<V>()] = k < ln ? (V)f.val[k0 + k] : (V)-0.0;
-        }
-        if (d) dd[i] = (V)d[r];
-      }
-      list[turn].push_back({(uint32_t)(base / 16), p, G,
-                            (uint32_t)(p % W) | (uint32_t)(m - 1) << 15 | (uint32_t)ke << 21 | (uint32_t)nc << 24});
-      turn = (turn + 1) % TP_NW;
-      ++ingroup;
-      p += m;
-    }
-  }
-  out.ngroups = G + 1;
-  out.hdr.clear();
-  out.first.clear();
-  for (const auto& q : list) {
-    out.first.push_back((int)out.hdr.size());
-    out.hdr.insert(out.hdr.end(), q.begin(), q.end());
-    for (int e = 0; e < 2; ++e) out.hdr.push_back({0, 0, out.ngroups, 0});
-  }
-  out.first.push_back((int)out.hdr.size());
-  out.bytes.resize(out.bytes.size() + 64, 0);  // (an ending header's row is read, and not used)
-  return true;
-}
 
 // --------------------------------------------------------------- kernels
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
