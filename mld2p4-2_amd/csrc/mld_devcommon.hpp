@@ -596,15 +596,24 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
 }
 
 // SELL, SELD operators whose values are few: packed words beside the arrays
-// (see sellp_kernel).  From 32768 rows, as the DIA classes: below, an operator
-// lies in the caches and its product takes the time of its gathers.  Tables of
-// more than 1024 values where 512 rows and more share one: loading the table
-// is then hidden by the other workgroups of the launch.
-constexpr int DICT_MIN_ROWS = 32768;
+// (see sellp_kernel).  From 32768 rows on: below, an operator lies in the caches
+// and its product takes the time of its gathers.  FP32 values, whose words save
+// 4 bytes of 8 instead of 8 of 12, from 98304 rows on: the table, which every
+// workgroup waits for, costs smaller launches more than that.  Level 1 below a
+// Poisson grid, V-cycles with l1-Jacobi 2/2, arrays -> words of one operator:
+// FP32 64 560 rows A 89.4 -> 91.1 us, R 91.2 -> 92.4; 82 658 rows A 107.3 ->
+// 110.8; 105 692 rows A 120.7 -> 121.6, R 122.8 -> 122.7; 129 684 rows A 120.2
+// -> 120.2, R 122.0 -> 119.6; 263 552 rows all three 184.4 -> 173.1.  FP64 64
+// 560 rows P 103.0 -> 96.3, R 101.4 -> 98.4, A 98.0 -> 98.6; 105 692 rows R
+// 137.7 -> 134.1.  Tables of more than 1024 values where 512 rows and more
+// share one: loading the table is then hidden by the other workgroups of the
+// launch.
+template <typename V>
+constexpr int dict_min_rows() { return sizeof(V) == 8 ? 32768 : 98304; }
 template <typename V>
 static void value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
   m.pk = nullptr;
-  if ((m.fmt != FMT_SELL && m.fmt != FMT_SELD) || m.nr < DICT_MIN_ROWS || m.stored < 1) return;
+  if ((m.fmt != FMT_SELL && m.fmt != FMT_SELD) || m.nr < dict_min_rows<V>() || m.stored < 1) return;
   int cb = 16;
   if (m.fmt == FMT_SELL)
     for (cb = 1; cb < 31 && ((int64_t)1 << cb) < m.nc; ++cb) {}
