@@ -63,9 +63,10 @@ class DevPrecT : public DevPrec {
       D.sweeps_pre = H.parms.sweeps_pre;
       D.sweeps_post = H.parms.sweeps_post;
       D.ml_cycle = H.parms.ml_cycle;
-      upload_smoother(H.smd, D.sm, p.dev_format);
+      const int sweeps = std::max(D.sweeps_pre, D.sweeps_post);
+      upload_smoother(H.smd, D.sm, p.dev_format, sweeps);
       D.has_sm2 = H.sm2a.allocated;
-      if (D.has_sm2) upload_smoother(H.smd2, D.sm2, p.dev_format);
+      if (D.has_sm2) upload_smoother(H.smd2, D.sm2, p.dev_format, sweeps);
       const size_t n = (size_t)D.n;
       D.x2l = ar_.alloc<V>(n); D.y2l = ar_.alloc<V>(n);
       D.tx = ar_.alloc<V>(n); D.ty = ar_.alloc<V>(n);
@@ -691,7 +692,8 @@ class DevPrecT : public DevPrec {
     HIPCHECK(hipGetLastError());
   }
 
-  void upload_smoother(const SmootherData& H, DSmoother<V>& S, int force) {
+  // sweeps: the level's; what no sweep of it reads gets no packed form
+  void upload_smoother(const SmootherData& H, DSmoother<V>& S, int force, int sweeps) {
     S.smoother = H.smoother;
     S.solver = H.solver;
     S.nnz_nd = H.nnz_nd;
@@ -722,10 +724,14 @@ class DevPrecT : public DevPrec {
                                                                                S.dv, S.ndd.val);
       }
       HIPCHECK(hipGetLastError());
-      dia_classes<V>(S.nd, S.dv, ar_, s_);
-      dia_classes<V>(S.ndd, S.dv, ar_, s_);
-      value_dictionary<V>(S.nd, ar_, s_);
-      value_dictionary<V>(S.ndd, ar_, s_);
+      if (sweeps >= 2) {
+        dia_classes<V>(S.ndd, S.dv, ar_, s_);
+        value_dictionary<V>(S.ndd, ar_, s_);
+      }
+      if (sweeps >= 3) {
+        dia_classes<V>(S.nd, S.dv, ar_, s_);
+        value_dictionary<V>(S.nd, ar_, s_);
+      }
     }
     if (H.solver == ILU_N || H.solver == GS || H.solver == BWGS) {
       S.l = upload_mat<V>(H.l, ar_, s_, 1, 1);  // CSR (rows summed in stored order)
