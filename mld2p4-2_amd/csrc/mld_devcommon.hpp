@@ -142,14 +142,26 @@ static inline void h2d_copy(void* dst, const void* src, size_t bytes, hipStream_
   host_to_device(dst, src, bytes, s);
 }
 
+// Device memory that was refused.
+struct NoRoom : DevError {
+  using DevError::DevError;
+};
 struct DevArena {
   std::vector<void*> ptrs;
   size_t bytes = 0;
+  size_t extra = 0;    // of these, in forms that a level can do without (optional_form)
+  int64_t room = -1;   // bytes that it may take (-1: what there is)
   template <typename T>
   T* alloc(size_t n) {
     if (n == 0) n = 1;
+    if (room >= 0 && bytes + n * sizeof(T) > (size_t)room) throw NoRoom("no room for an optional form");
     void* p = nullptr;
-    HIPCHECK(hipMalloc(&p, n * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, n * sizeof(T));
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // not the next launch's error
+      throw NoRoom("hipMalloc of " + std::to_string(n * sizeof(T)) + " bytes: " + hipGetErrorString(e));
+    }
+    HIPCHECK(e);
     ptrs.push_back(p);
     bytes += n * sizeof(T);
     return (T*)p;
@@ -164,6 +176,36 @@ struct DevArena {
     for (void* p : ptrs) (void)hipFree(p);
   }
 };
+
+// A form that products can do without (row classes, value tables, packed
+// factors, dense tails): f(arena) puts its memory into an arena of its own,
+// which ar takes over when f returns true; where memory is refused, the form is
+// left out and what was there before stays in use (f sets nothing before it has
+// all of its memory).  It is also left out where the card would have less left
+// than ar holds by then: transposes, vectors and block engines come later and
+// need their room.  MLD_EXTRA_MB: at most that much for all such forms of ar.
+template <class F>
+static bool optional_form(DevArena& ar, F f) {
+  size_t avail = 0, total = 0;
+  HIPCHECK(hipMemGetInfo(&avail, &total));
+  int64_t room = (int64_t)avail - (int64_t)ar.bytes;
+  if (const char* e = std::getenv("MLD_EXTRA_MB"))
+    room = std::min<int64_t>(room, (int64_t)std::atoi(e) * 1000000 - (int64_t)ar.extra);
+  if (room <= 0) return false;
+  DevArena own;
+  own.room = room;
+  try {
+    if (!f(own)) return false;
+  } catch (const NoRoom&) {
+    if (std::getenv("MLD_VERBOSE")) std::fprintf(stderr, "[mld] an optional form left out: no room\n");
+    return false;
+  }
+  ar.ptrs.insert(ar.ptrs.end(), own.ptrs.begin(), own.ptrs.end());
+  own.ptrs.clear();
+  ar.bytes += own.bytes;
+  ar.extra += own.bytes;
+  return true;
+}
 
 static inline int nblk(int64_t n) { return (int)((n + BS - 1) / BS); }
 
@@ -504,9 +546,7 @@ struct gather_x<GatherX<V, XT>> : std::true_type {};
 // -> 3.6 us.
 constexpr double DIACLS_MIN_BYTES = 7e6;
 template <typename V>
-static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
-  m.cls = nullptr;
-  if (m.fmt != FMT_DIA || m.w < 1 || (d && m.w > 7) || (double)m.nr * m.w * sizeof(V) < DIACLS_MIN_BYTES) return;
+static bool form_dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
   struct Work {  // one allocation; from tab on copied back together
     unsigned long long keys[DIACLS_SLOTS];
     int rep[DIACLS_SLOTS], num[DIACLS_SLOTS];
@@ -524,7 +564,7 @@ static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
   int n = 0;
   HIPCHECK(hipMemcpyAsync(&n, &w->many, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHECK(hipStreamSynchronize(s));
-  if (n > 256) return;
+  if (n > 256) return false;
   uint8_t* cls = ar.alloc<uint8_t>((size_t)m.nr);
   dia_class_number<V><<<1, BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->rep, w->num, w->tab);
   dia_class_rows<V><<<nblk(m.nr), BS, 0, s>>>(m.nr, m.w, m.val, d, w->keys, w->num, w->tab, cls, &w->many);
@@ -534,21 +574,29 @@ static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
   const size_t skip = offsetof(Work, tab);
   HIPCHECK(hipMemcpyAsync((char*)&host + skip, (char*)w + skip, sizeof(Work) - skip, hipMemcpyDeviceToHost, s));
   HIPCHECK(hipStreamSynchronize(s));
-  if (host.many > 256) return;
+  if (host.many > 256) return false;
   // the commonest class: the majority of the sampled rows
   int count[256] = {}, best = host.at[0];
   for (int q = 0; q < DIACLS_NS; ++q)
     if (++count[host.at[q]] > count[best]) best = host.at[q];
-  m.ctab = ar.alloc<V>(8 * 256);
-  HIPCHECK(hipMemcpyAsync(m.ctab, w->tab, sizeof(host.tab), hipMemcpyDeviceToDevice, s));
+  V* ctab = ar.alloc<V>(8 * 256);
+  HIPCHECK(hipMemcpyAsync(ctab, w->tab, sizeof(host.tab), hipMemcpyDeviceToDevice, s));
   HIPCHECK(hipStreamSynchronize(s));
   m.cls = cls;
+  m.ctab = ctab;
   m.ctab_d = d != nullptr;
   m.cdef.c = best;
   m.cdef.n = n;
   for (int k = 0; k < 8; ++k) m.cdef.v[k] = host.tab[8 * best + k];
   if (std::getenv("MLD_VERBOSE"))
     std::fprintf(stderr, "[mld] %d x %d operator (DIA): %d distinct rows\n", m.nr, m.nc, n);
+  return true;
+}
+template <typename V>
+static void dia_classes(DMat<V>& m, const V* d, DevArena& ar, hipStream_t s) {
+  m.cls = nullptr;
+  if (m.fmt != FMT_DIA || m.w < 1 || (d && m.w > 7) || (double)m.nr * m.w * sizeof(V) < DIACLS_MIN_BYTES) return;
+  optional_form(ar, [&](DevArena& o) { return form_dia_classes(m, d, o, s); });
 }
 
 // DIA launch (with its final reduction when K > 0): two adjacent rows per
@@ -611,9 +659,7 @@ static void dia_launch(const DMat<V>& m, G g, E e, hipStream_t s, Red red) {
 template <typename V>
 constexpr int dict_min_rows() { return sizeof(V) == 8 ? 32768 : 98304; }
 template <typename V>
-static void value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
-  m.pk = nullptr;
-  if ((m.fmt != FMT_SELL && m.fmt != FMT_SELD) || m.nr < dict_min_rows<V>() || m.stored < 1) return;
+static bool form_value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
   int cb = 16;
   if (m.fmt == FMT_SELL)
     for (cb = 1; cb < 31 && ((int64_t)1 << cb) < m.nc; ++cb) {}
@@ -632,19 +678,29 @@ static void value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
   int n = 0;
   HIPCHECK(hipMemcpyAsync(&n, &w->many, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHECK(hipStreamSynchronize(s));
-  if (n < 1 || n > std::min(DICT_MAX, std::max(1024, m.nr / 512)) || (int64_t)n > ((int64_t)1 << (32 - cb))) return;
-  m.ptab = ar.alloc<V>(n);
-  m.pk = ar.alloc<uint32_t>((size_t)m.stored);
-  m.pnt = n;
-  m.pcb = cb;
-  dict_number<V><<<1, BS, 0, s>>>(w->keys, w->num, m.ptab);
+  if (n < 1 || n > std::min(DICT_MAX, std::max(1024, m.nr / 512)) || (int64_t)n > ((int64_t)1 << (32 - cb)))
+    return false;
+  V* ptab = ar.alloc<V>(n);
+  uint32_t* pk = ar.alloc<uint32_t>((size_t)m.stored);
+  dict_number<V><<<1, BS, 0, s>>>(w->keys, w->num, ptab);
   dict_pack<V><<<blocks(m.stored), BS, 0, s>>>(m.stored, m.val, m.ja, m.fmt == FMT_SELD ? m.dja : nullptr, w->keys,
-                                               w->num, cb, m.pk);
+                                               w->num, cb, pk);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));  // before tmp is released
+  m.ptab = ptab;
+  m.pk = pk;
+  m.pnt = n;
+  m.pcb = cb;
   if (std::getenv("MLD_VERBOSE"))
     std::fprintf(stderr, "[mld] %d x %d operator (%s): %d distinct values\n", m.nr, m.nc,
                  m.fmt == FMT_SELL ? "SELL" : "SELD", n);
+  return true;
+}
+template <typename V>
+static void value_dictionary(DMat<V>& m, DevArena& ar, hipStream_t s) {
+  m.pk = nullptr;
+  if ((m.fmt != FMT_SELL && m.fmt != FMT_SELD) || m.nr < dict_min_rows<V>() || m.stored < 1) return;
+  optional_form(ar, [&](DevArena& o) { return form_value_dictionary(m, o, s); });
 }
 template <typename C, typename V, class G, class E>
 static void sellp_launch(const DMat<V>& m, G g, E e, hipStream_t s) {

@@ -158,8 +158,12 @@ class DevPrecT : public DevPrec {
   void build_tail() {
     tail_lev_ = -1;
     tail_b_ = nullptr;
+    tail_k_ = false;
+    optional_form(ar_, [&](DevArena& o) { return form_tail(o); });
+  }
+  bool form_tail(DevArena& own) {
     if (const char* e = std::getenv("MLD_DENSE_TAIL"))
-      if (e[0] == '0') return;
+      if (e[0] == '0') return false;
     const int nlev = (int)L_.size();
     const double few = 16.0 * (double)hprec_->precv[0].a.nnz();
     auto fits = [&](int l) {
@@ -173,17 +177,17 @@ class DevPrecT : public DevPrec {
     };
     int l = 1;
     while (l < nlev && !fits(l)) ++l;
-    if (l >= nlev) return;
+    if (l >= nlev) return false;
     bool kc = false;
     for (int k = l; k < nlev; ++k) kc = kc || L_[k].ml_cycle == KCYCLE || L_[k].ml_cycle == KCYCLESYM;
-    tail_k_ = kc;
     if (kc) l = nlev - 1;  // fits, the levels shrink
-    if (kc && !fits(l)) return;
+    if (kc && !fits(l)) return false;
     DLevel<V>& D = L_[l];
-    if (l == nlev - 1 && (D.sm.solver == DENSE_LU || D.sm.smoother == NOPREC)) return;
-    if (kc && D.sm.solver != ILU_N && D.sm.solver != GS && D.sm.solver != BWGS) return;
+    if (l == nlev - 1 && (D.sm.solver == DENSE_LU || D.sm.smoother == NOPREC)) return false;
+    if (kc && D.sm.solver != ILU_N && D.sm.solver != GS && D.sm.solver != BWGS) return false;
     const int n = D.n, ld = (n + 63) / 64 * 64;
     DevArena tmp;
+    tmp.room = own.room;
     std::vector<tail::Lev> T(nlev - l);
     auto smoother = [&](const SmootherData& h, const DSmoother<V>& d) {
       tail::Sm t;
@@ -232,15 +236,17 @@ class DevPrecT : public DevPrec {
     tail::Cycle cyc(T, n, ld, s_);
     if (!cyc.run()) {  // the cycle stays as it is
       HIPCHECK(hipStreamSynchronize(s_));
-      return;
+      return false;
     }
-    V* B = ar_.alloc<V>((size_t)n * ld);
+    V* B = own.alloc<V>((size_t)n * ld);
     tail::mstore_kernel<V><<<dim3(n, (ld + 255) / 256), 256, 0, s_>>>(n, ld, T[0].y, ld, B);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s_));
     tail_b_ = B;
     tail_ld_ = ld;
     tail_lev_ = l;
+    tail_k_ = kc;
+    return true;
   }
   // The transposed cycle below the tail level as one product with B^T: 50 us
   // of a 72^3 FP32 cycle (six launches, one a substitution in one workgroup)
@@ -252,7 +258,9 @@ class DevPrecT : public DevPrec {
   // transposed operators are there.
   void build_tail_t() {
     tail_bt_ = nullptr;
-    if (tail_lev_ < 0) return;
+    if (tail_lev_ >= 0) optional_form(ar_, [&](DevArena& o) { return form_tail_t(o); });
+  }
+  bool form_tail_t(DevArena& own) {
     DLevel<V>& D = L_[tail_lev_];
     const int n = D.n;
     std::vector<V> x(n), y(n), z(n);
@@ -261,11 +269,11 @@ class DevPrecT : public DevPrec {
       h = h * 6364136223846793005ull + 1442695040888963407ull;
       v = (V)((double)(int64_t)h * 0x1p-63);
     }
+    V* bt = own.alloc<V>((size_t)n * tail_ld_);
     HIPCHECK(hipMemcpyAsync(D.x2l, x.data(), n * sizeof(V), hipMemcpyHostToDevice, s_));
     HIPCHECK(hipStreamSynchronize(s_));
-    if (inner_ml_aply(tail_lev_, 'T') != 0) return;
+    if (inner_ml_aply(tail_lev_, 'T') != 0) return false;
     HIPCHECK(hipMemcpyAsync(y.data(), D.y2l, n * sizeof(V), hipMemcpyDeviceToHost, s_));
-    V* bt = ar_.alloc<V>((size_t)n * tail_ld_);
     const dim3 g((tail_ld_ + 31) / 32, (n + 31) / 32);
     transpose_kernel<V><<<g, dim3(32, 8), 0, s_>>>(n, tail_ld_, tail_b_, bt);
     tail_gemv(D, bt);
@@ -275,9 +283,11 @@ class DevPrecT : public DevPrec {
     for (int i = 0; i < n; ++i) {
       dmax = std::max(dmax, std::fabs((double)y[i] - (double)z[i]));
       ymax = std::max(ymax, std::fabs((double)y[i]));
-      if (!std::isfinite((double)y[i]) || !std::isfinite((double)z[i])) return;
+      if (!std::isfinite((double)y[i]) || !std::isfinite((double)z[i])) return false;
     }
-    if (dmax <= (sizeof(V) == 8 ? 1e-13 : 5e-6) * ymax) tail_bt_ = bt;
+    if (!(dmax <= (sizeof(V) == 8 ? 1e-13 : 5e-6) * ymax)) return false;
+    tail_bt_ = bt;
+    return true;
   }
   // y2l = B x2l at the tail level
   void tail_gemv(DLevel<V>& D, const V* B) {
@@ -805,29 +815,40 @@ class DevPrecT : public DevPrec {
     const double* d = H.dv.empty() ? nullptr : H.dv.data();
     if (H.solver != BWGS && !tp::tp_pack(H.l, H.lsched_ptr, H.lsched_rows, ilu ? nullptr : d, pl)) return;
     if (H.solver != GS && !tp::tp_pack(H.u, H.usched_ptr, H.usched_rows, d, pu)) return;
-    std::vector<int> pos(n), idx(n);
-    auto up = [&](const tp::Packed<V>& f, typename DSmoother<V>::PackedTri& t) {
-      for (int p = 0; p < n; ++p) pos[f.rows[p]] = p;
-      t.pk = ar_.upload(f.bytes.data(), f.bytes.size(), s_);
-      t.hdr = ar_.upload((const int*)f.hdr.data(), f.hdr.size() * 4, s_);
-      t.first = ar_.upload(f.first.data(), f.first.size(), s_);
-      t.in = ar_.upload(f.rows.data(), f.rows.size(), s_);
-      t.pos = ar_.upload(pos.data(), pos.size(), s_);
-      t.ngroups = f.ngroups;
-      HIPCHECK(hipStreamSynchronize(s_));
-    };
-    if (pl.ngroups) up(pl, S.lp);
-    if (ilu) {  // pos holds L's positions
-      for (int p = 0; p < n; ++p) idx[p] = pos[pu.rows[p]];
-      S.ulin = ar_.upload(idx.data(), idx.size(), s_);
-      HIPCHECK(hipStreamSynchronize(s_));
-    }
-    if (pu.ngroups) up(pu, S.up);
-    S.tpa = ar_.alloc<V>(n);
-    S.tpb = ar_.alloc<V>(n);
-    if (std::getenv("MLD_VERBOSE"))
-      std::fprintf(stderr, "[mld] %d-row factors packed for one workgroup: %d and %d groups, %zu and %zu level sets\n",
-                   n, pl.ngroups, pu.ngroups, H.lsched_ptr.size() - 1, H.usched_ptr.size() - 1);
+    optional_form(ar_, [&](DevArena& own) {
+      std::vector<int> pos(n), idx(n);
+      typename DSmoother<V>::PackedTri lp, up;
+      int* ulin = nullptr;
+      auto put = [&](const tp::Packed<V>& f, typename DSmoother<V>::PackedTri& t) {
+        for (int p = 0; p < n; ++p) pos[f.rows[p]] = p;
+        t.pk = own.upload(f.bytes.data(), f.bytes.size(), s_);
+        t.hdr = own.upload((const int*)f.hdr.data(), f.hdr.size() * 4, s_);
+        t.first = own.upload(f.first.data(), f.first.size(), s_);
+        t.in = own.upload(f.rows.data(), f.rows.size(), s_);
+        t.pos = own.upload(pos.data(), pos.size(), s_);
+        t.ngroups = f.ngroups;
+        HIPCHECK(hipStreamSynchronize(s_));
+      };
+      if (pl.ngroups) put(pl, lp);
+      if (ilu) {  // pos holds L's positions
+        for (int p = 0; p < n; ++p) idx[p] = pos[pu.rows[p]];
+        ulin = own.upload(idx.data(), idx.size(), s_);
+        HIPCHECK(hipStreamSynchronize(s_));
+      }
+      if (pu.ngroups) put(pu, up);
+      V* tpa = own.alloc<V>(n);
+      V* tpb = own.alloc<V>(n);
+      S.lp = lp;
+      S.up = up;
+      S.ulin = ulin;
+      S.tpa = tpa;
+      S.tpb = tpb;
+      if (std::getenv("MLD_VERBOSE"))
+        std::fprintf(stderr,
+                     "[mld] %d-row factors packed for one workgroup: %d and %d groups, %zu and %zu level sets\n", n,
+                     pl.ngroups, pu.ngroups, H.lsched_ptr.size() - 1, H.usched_ptr.size() - 1);
+      return true;
+    });
   }
   static constexpr int TP_MIN_ROWS = 128;
   static int tp_blocks(int n) { return (n + 255) / 256; }
