@@ -285,7 +285,11 @@ class DevPrecT : public DevPrec {
       ymax = std::max(ymax, std::fabs((double)y[i]));
       if (!std::isfinite((double)y[i]) || !std::isfinite((double)z[i])) return false;
     }
-    if (!(dmax <= (sizeof(V) == 8 ? 1e-13 : 5e-6) * ymax)) return false;
+    const bool same = dmax <= (sizeof(V) == 8 ? 1e-13 : 5e-6) * ymax;
+    if (std::getenv("MLD_VERBOSE"))
+      std::fprintf(stderr, "[mld] transposed dense tail of %d rows: off by %.1e of its largest value, %s\n", n,
+                   dmax / ymax, same ? "used" : "not used");
+    if (!same) return false;
     tail_bt_ = bt;
     return true;
   }
