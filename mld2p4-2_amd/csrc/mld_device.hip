@@ -1743,7 +1743,11 @@ class DevPrecT : public DevPrec {
 // Krylov solvers, all vectors device-resident in FP64.  The preconditioner
 // is applied through the same apply() the C-ABI exposes (the psb_krylov ->
 // prec%apply call site).  Convergence test (istop = 2): ||r||_2/||b||_2 <= eps
-// after each iteration; one 8-byte device-to-host read per iteration.
+// after each iteration.  The reduction that ends an iteration (CG, FCG; five
+// times an iteration in BiCGStab) stores the scalar slots and a sequence
+// number in pinned host memory, which the host polls (read_scal).  The next
+// application may be enqueued by then; where the solve ends instead, it is
+// waited for before the call returns and its result is not used.
 // ---------------------------------------------------------------------------
 template <typename V>
 int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int itmax, int istop, int* iter,
