@@ -759,7 +759,8 @@ def main():
             traffic = None
     copy_gbs = copy_bandwidth(torch)
     log(f"device-to-device copy of 2 GiB (HIP runtime copy kernel): {copy_gbs:.0f} GB/s")
-    roofline = {"bound": "hbm", "kernel": f"fine-level {dom} (level 1 of {p.nlev}), launches inside V-cycles",
+    launches = "inside V-cycles" if dom == "residual" else "one after the other"
+    roofline = {"bound": "hbm", "kernel": f"fine-level {dom} (level 1 of {p.nlev}), launches {launches}",
                 "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic, "algorithmic_bytes": int(by), "avg_ms": round(ms, 5),
