@@ -9,18 +9,22 @@
 // what happens between two barriers: the slices of a level set, each on a
 // wavefront of its own.  Slices go to the TP_NW wavefronts in turn, so every
 // wavefront has the time of several groups to bring its next slice's entries
-// from memory into registers (12 wavefronts with up to 10 KB each in flight;
-// one CU streams about 100 GB/s that way), and to sum, in order, the leading
-// entries that no row of the group before theirs is gathered for (a row's
-// latest neighbours are mostly its last ones).  Between two barriers stand
-// only the remaining gathers, products and additions and one LDS store.
+// from memory into registers (12 wavefronts with up to 10 KB each in flight),
+// and to sum, in order, the leading entries that no row of the group before
+// theirs is gathered for (a row's latest neighbours are mostly its last ones).
+// Between two barriers stand only the remaining gathers, products and additions
+// and one LDS store.
 //
 // FP64 on MI355X, per level set: Gauss-Seidel on a 301 x 301 grid (150 rows of
-// 2 entries) 1.65 -> 0.35 us, its first coarse level (32 rows of 4) 1.35 ->
-// 0.25 us; ILU(0) on the first coarse level of a 96^3 grid (127 rows of 15)
-// 1.53 -> 0.64 us, and of a 64^2 grid in one workgroup with row lists
-// (trsv_run_kernel) 1.0 -> 0.25 us.  What is left is the chain: an LDS store,
-// barrier and read take 134-176 cycles, an addition 8, a division 76.
+// 2 entries) 1.65 -> 0.34 us, its first coarse level (32 rows of 4) 1.35 ->
+// 0.28 us; ILU(0) on the first coarse level of a 96^3 grid (127 rows of 15)
+// 1.53 -> 0.70 us forward and 0.50 backward, and of a 64^2 grid in one workgroup
+// with row lists (trsv_run_kernel) 1.0 -> 0.28 us.  What is left is the chain: an
+// LDS store, barrier and read take 134-176 cycles, an addition 8, a division 76;
+// the wavefronts wait for 82 % of their cycles.  Not the bytes: 20.7 MB of that
+// factor pass at 35-50 GB/s, where one CU streams 95-117.  The sums ahead gain
+// nothing there (forward 588 us with 7.6 of 18.8 entries per row ahead, 418 with
+// none) nor on the 2-D grids (1 %).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -121,7 +125,8 @@ __global__ __launch_bounds__(TP_T, 1) void tripack_kernel(int ngroups, const uns
 #pragma unroll
     for (int k = 0; k < C; ++k) acc = acc + ev[k / VPC][k % VPC] * t[k];
     // keeps the cases of the switch apart: with their common ends merged the
-    // compiler (ROCm 7.2) leaves columns of the longer case undefined
+    // compiler (ROCm 7.2) has left columns of the longer case undefined
+    // (tests/test_gpu_packed_cases.py runs every pair of cases)
     asm volatile("; ahead %0" ::"n"(C));
   };
   // The rest of the slice: what can be done before the barrier is, so that
