@@ -250,9 +250,9 @@ int mldhip_get_tri_levels(mldhip_prec* p, int lev, int which, int* nl_lower, int
 /* First level of the dense tail (the untransposed cycle on levels lev ..
  * nlev-1 applied as one dense product, formed at smoothers_build), or -1 when
  * the cycle runs level by level (MLD_DENSE_TAIL=0 at build, no small level
- * below the fine level, a K-cycle there, no memory for it).  Small: at most 1024 rows, or n^2 <=
- * 16 nnz(A_1) and n^2 values in at most 48 MB (134 MB above triangular
- * solves).  No reference counterpart. */
+ * below the fine level, a K-cycle there, no memory for it).  Small: at most
+ * 1024 rows, or n^2 <= 16 nnz(A_1) and n^2 values in at most 48 MB (134 MB above
+ * triangular solves).  No reference counterpart. */
 int mldhip_get_dense_tail(mldhip_prec* p, int* lev);
 /* Operator complexity sum nnz(A_l)/nnz(A_1) (mld_d_prec_type.f90:465-497). */
 int mldhip_get_complexity(mldhip_prec* p, double* cplx);

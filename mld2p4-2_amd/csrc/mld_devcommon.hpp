@@ -284,7 +284,10 @@ static FmtChoice choose_format(const HCsr& h, int force) {
   // for rows of 8 entries or more while one lane each leaves most of the chip
   // without a wavefront and makes a long chain of each row: 6251 rows of 62
   // entries FP32 13.2 -> 4.6 us, of 215 entries (a restriction) 52 -> 6.9
-  // us; 7809 rows of 29 entries FP64 7.6-11 -> 3.7 us
+  // us; 7809 rows of 29 entries FP64 7.6-11 -> 3.7 us.  Residuals of 4096 to
+  // 32000 uneven rows of 8 to 60 entries, both types: 4096 rows of 8 FP64 4.5 ->
+  // 3.4 us, of 60 10.3 -> 2.8; the least gain at the line, 32000 rows of 60 FP64
+  // 13.6 -> 11.2 us (from 32768 rows on the tuner times both)
   if (h.nr >= 4096 && !(avg >= 8.0 && h.nr < SELL_FULL_ROWS)) { c.fmt = FMT_SELL; return c; }
   return c;
 }

@@ -139,7 +139,10 @@ class DevPrecT : public DevPrec {
   // them stays a small part of the cycle's traffic, and take at most
   // DENSE_TAIL_BYTES (Jacobi-type smoothers: about 30 us level by level; with
   // 82 MB, 3195 rows in FP64 below a 101^3 grid, a V-cycle takes 186 us
-  // against 184, with 36 MB, below 93^3, a CG iteration 214 against 229) or
+  // against 184, with 36 MB, below 93^3, a CG iteration 214 against 229; V-cycles
+  // level by level -> as a product: FP64 81^3 (17 MB) 123 -> 107 us, 89^3 (39 MB)
+  // 127 -> 118, FP32 95^3 (29 MB) 123 -> 111, 101^3 (41 MB) 127 -> 121; 2-D
+  // Jacobi 260^2 75 -> 60, 340^2 71 -> 65) or
   // DENSE_TAIL_BYTES_TRI where a level has triangular solves (2349 rows below
   // a 96^3 grid with ILU(0): 3.3 ms per cycle in one workgroup, 1.2 ms packed,
   // 10 us as one product).
