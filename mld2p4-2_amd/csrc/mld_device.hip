@@ -129,8 +129,8 @@ class DevPrecT : public DevPrec {
   // Dense tail: from a level l >= 1 on, the untransposed cycle on levels
   // l .. nlev-1 is a fixed linear operator B_l of x2l (no K-cycle there),
   // formed once here and applied afterwards as one dense product y2l = B_l
-  // x2l: about ten launches of a few microseconds each become one.  'T'
-  // applications keep the level-by-level cycle.  Not taken when that level is
+  // x2l: about ten launches of a few microseconds each become one
+  // ('T': see build_tail_t).  Not taken when that level is
   // a coarsest level already solved by one dense product (DENSE_LU), nor with
   // MLD_DENSE_TAIL=0.  Same operator; the sums of the product are rounded in
   // another order.

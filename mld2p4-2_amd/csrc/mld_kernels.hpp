@@ -1100,8 +1100,8 @@ __global__ __launch_bounds__(BS) void axpby_kernel(int n, V a, const V* __restri
   else y[i] = a * x[i] + b * y[i];
 }
 
-// Elements per thread of the streaming reduction kernels (each is followed
-// by finalize_kernel over its red_blocks(n) partials).
+// Elements per thread of the streaming reduction kernels (red_blocks(n) partial
+// sums each, added as block_partials says).
 constexpr int RED_EPT = 2;
 __host__ __device__ constexpr int red_blocks(int n) { return (n + BS * RED_EPT - 1) / (BS * RED_EPT); }
 
