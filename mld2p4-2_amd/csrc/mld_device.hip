@@ -1715,6 +1715,7 @@ class DevPrecT : public DevPrec {
     for (unsigned k = 1; __atomic_load_n(q, __ATOMIC_ACQUIRE) != seq_; ++k) {
       __builtin_ia32_pause();
       if (k % 4096 == 0) {
+        no_capture();  // (its launches do not run, so nothing would ever arrive)
         const hipError_t e = hipStreamQuery(s_);
         if (e == hipErrorNotReady) continue;
         HIPCHECK(e);
@@ -1724,6 +1725,12 @@ class DevPrecT : public DevPrec {
     }
     check_abort();
     return hscal_[slot];
+  }
+  // what reads scalars on the host cannot be captured into a graph
+  void no_capture() {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    HIPCHECK(hipStreamIsCapturing(s_, &st));
+    if (st != hipStreamCaptureStatusNone) throw DevError("solves and K-cycles read scalars: not under graph capture");
   }
   // a sync-free substitution that stopped waiting (see trsv_sf_kernel)
   void check_abort() {
@@ -1758,6 +1765,7 @@ int DevPrecT<V>::krylov(int method, const double* b, double* x, double eps, int 
   HIPCHECK(hipSetDevice(device_));
   if (istop != 2) return E_UNSUPPORTED;
   if (trans != 'N' && trans != 'T') return E_BAD_ARG;
+  no_capture();
   const int n = n0_;
   if (trans == 'T') {
     // adjoint system A^T x = b with M^T: transposed operators of every level
